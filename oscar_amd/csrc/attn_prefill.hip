@@ -13,16 +13,9 @@
 //                        when the seat's owner tag matches, prepare_kv.py:77) into a
 //                        caller-provided bf16 workspace, once per call: every query
 //                        tile of a long chunk reuses them;
-//   prefill_kernel       flash attention over [workspace history | current chunk].
-//                        A workgroup of four waves owns 128 query rows (tokens x heads
-//                        of one KV head, GQA packed; Q^T operands in LDS).  Key tiles of
-//                        32 are double-buffered in LDS: each thread prefetches its
-//                        share of tile t+2 into registers while tile t is computed, so
-//                        one barrier per tile separates the buffers.  Per wave:
-//                        S^T = K Q^T (v_mfma_f32_32x32x16_bf16 / _f16), online softmax
-//                        in fp32 (log2 domain) with a lazy reference max, O^T += V^T P^T
-//                        on v_mfma_f32_32x32x16_f16 (P and V in fp16, see kVShift) with
-//                        V^T read from LDS by ds_read_b64_tr_b16.
+//   prefill_kernel       flash attention over [workspace history | current chunk]: see there.
+#include <type_traits>
+
 #include "common.h"
 
 namespace oscar {
@@ -35,8 +28,9 @@ constexpr int kKeys = 32;
 constexpr int kRows = 128;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-constexpr float kLazy = 8.f;  // max drift (log2 units) before O is rescaled
-constexpr int kQK = 4;        // QK K-steps whose LDS operands are read together
+constexpr int kLazy = 10;     // log2 of the largest row sum of a tile's probabilities before O is rescaled
+// workgroups per CU the register budget of prefill_kernel<D, ., NB> is set for
+constexpr int prefill_wgs(int D, int NB) { return D == 256 ? 1 : 2; }
 // PV runs on v_mfma_f32_32x32x16_f16 with P and V in fp16 for both query dtypes.  bf16
 // V values (8-bit significands) are held as fp16(v * 2^-kVShift): exact for |v| from
 // 2^-6 up to 2^23 (below, within 2^-17 absolutely), and O is scaled back by 2^kVShift.
@@ -53,12 +47,6 @@ __device__ __forceinline__ unsigned hist_bits(float x) {
   if constexpr (QT == OSCAR_F16) return __half_as_ushort(h);
   else return f32_to_bf16_bits(__half2float(h));
 }
-// 16-bit bits of x in the query dtype (RNE)
-template <int QT>
-__device__ __forceinline__ unsigned q_bits(float x) {
-  if constexpr (QT == OSCAR_F16) return f32_to_f16_bits(x);
-  else return f32_to_bf16_bits(x);
-}
 // the PV operand bits of a value v already in the query dtype: fp16 as it is; a bf16
 // value scaled by 2^-kVShift into fp16 (exact, see kVShift)
 template <int QT>
@@ -66,16 +54,43 @@ __device__ __forceinline__ unsigned pv_bits(float v) {
   if constexpr (QT == OSCAR_F16) return f32_to_f16_bits(v);
   else return f32_to_f16_bits(v * (1.f / (1 << kVShift)));
 }
+// two packed bf16 values to their PV operand bits: fp16(v * 2^-kVShift), one
+// mixed-precision multiply-add each
+__device__ __forceinline__ unsigned pv_pair(unsigned w) {
+  constexpr float k = 1.f / (1 << kVShift);
+  unsigned d;
+  asm volatile("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(d) : "v"(w << 16), "s"(k));
+  asm volatile("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(d) : "v"(w & 0xffff0000u), "s"(k));
+  return d;
+}
 template <int QT> struct QVec { typedef bf16x8 type; typedef bf16x2 pair; typedef __bf16 elem; };
 template <> struct QVec<OSCAR_F16> { typedef f16x8 type; typedef f16x2 pair; typedef _Float16 elem; };
+
+// four consecutive output elements from element i: the query dtype without a history
+// (original domain), else fp32 rotated.  One store each, at whatever alignment the
+// caller's output has.
+template <int QT>
+__device__ __forceinline__ void store_out(const oscar_prefill_args_v1& A, int64_t i, f32x4 v) {
+  typedef u32x2 __attribute__((aligned(2))) u32x2_any;
+  typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+  if (A.history != 0) {
+    *(f32x4_any*)((float*)A.out + i) = v;
+  } else {
+    using Q2 = typename QVec<QT>::pair;
+    *(u32x2_any*)((uint16_t*)A.out + i) =
+        u32x2{__builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{v[0], v[1]}, Q2)),
+              __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{v[2], v[3]}, Q2))};
+  }
+}
 
 // ---- balanced split of the key ranges (a workspace of oscar_prefill_workspace_bytes_v2)
 // Query tile qt (kRows GQA rows) sees key tiles [0, kt(qt)), kt growing with qt under
 // the causal mask.  One workgroup per tile leaves the chip unbalanced: the continuation
-// of 15360 + 9256 tokens is 441 tiles of 481..771 key tiles on 256 CUs (1.7 rounds), a
+// of 15360 + 9256 tokens is 441 tiles of 481..771 key tiles on 256 CUs, a
 // fresh 2048-token prefill 96 tiles (a third of the CUs).  The key range of a tile is
-// instead cut into chunks of U key tiles (c U .. (c + 1) U), U about the work of half a
-// CU, and every chunk is a workgroup ("unit"); a tile with more than one chunk writes
+// instead cut into chunks of U key tiles (c U .. (c + 1) U), U a little over the work of
+// half a CU, and every chunk is a unit (a workgroup takes one, or the same chunk of two
+// neighbouring tiles); a tile with more than one chunk writes
 // normalised partials + log2 LSEs, and prefill_merge_kernel combines them (FP32 LSE
 // merge).  Units are numbered chunk-major, heaviest tile first within a chunk index,
 // so the large units are dispatched first: the tiles that have a chunk c are the
@@ -101,6 +116,7 @@ struct PrefillParams {
   int ntq;             // query tiles
   int qmin1;           // first tile with two chunks (the split tiles are qt >= qmin1)
   int base[kMaxChunks + 1];
+  int pbase[kMaxChunks + 1];  // first workgroup of chunk class c when a workgroup takes two query tiles
   float* part_o;       // [slot][Hk][kRows][D] normalised partial O of the split tiles' chunks
   float* part_lse;     // [slot][Hk][kRows] log2-domain LSE of each partial
 };
@@ -123,6 +139,10 @@ SplitPlan plan_split(int64_t hist, int64_t n, int64_t qtok, int64_t hk) {
   for (int64_t qt = 0; qt < ntq; ++qt) work += kt(qt);
   const int64_t kmax = kt(ntq - 1);
   int64_t U = (work * hk + kSplitCUs * kUnitsPerCU - 1) / (kSplitCUs * kUnitsPerCU);
+  // a little over half a CU's share: the longest units, dispatched first, then fit one round
+  // of the chip with the shorter ones filling the rest.  15360 + 9256 tokens: 1231 us;
+  // exactly the share 1287 us, two thirds of it 1391 us, half of it 1300 us.
+  if (U + U / 32 + 3 < kmax) U += U / 32 + 3;
   if (U < kMinChunkTiles) U = kMinChunkTiles;
   if ((kmax + U - 1) / U > kMaxChunks) U = (kmax + kMaxChunks - 1) / kMaxChunks;
   const int64_t chunks = (kmax + U - 1) / U;
@@ -215,265 +235,559 @@ __global__ __launch_bounds__(256) void history_bf16_kernel(PrefillParams P) {
   }
 }
 
-template <int D, int QT>
-__global__ __launch_bounds__(kThreads, 1) void prefill_kernel(PrefillParams P) {
+// One 16-byte-per-lane LDS DMA: lane l's 16 bytes at `addr` land at LDS offset lds + 16 l.
+// The wait is the caller's (vmcnt): the builtin form would make the compiler drain every
+// load before each later LDS read.
+__device__ __forceinline__ void dma16(unsigned lds, const void* addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(addr) : "memory");
+}
+
+// the same with a uniform base and a 32-bit byte offset
+__device__ __forceinline__ void dma16(unsigned lds, uint64_t base, unsigned voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+}
+
+// Every wave's LDS traffic is done and all but the last PENDING of this wave's DMA
+// instructions have landed, then the workgroup barrier.
+template <int PENDING>
+__device__ __forceinline__ void tile_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PENDING) : "memory");
+}
+
+// S (+)= K Q^T with S in VGPRs.  The builtin would put every accumulator of a kernel of
+// more than 256 registers into AGPRs, and the softmax would copy S out; O stays there.
+template <int QT, bool FIRST, class QV>
+__device__ __forceinline__ void mfma_qk(f32x16& S, QV k, QV q) {
+  if constexpr (QT == OSCAR_F16) {
+    if constexpr (FIRST) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(S) : "v"(k), "v"(q));
+    else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(S) : "v"(k), "v"(q));
+  } else {
+    if constexpr (FIRST) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(S) : "v"(k), "v"(q));
+    else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(S) : "v"(k), "v"(q));
+  }
+}
+
+// o *= f with o in an AGPR.  Written out so that O has no other home than the AGPRs: an
+// ordinary product makes the compiler move all of O to VGPRs and back in every iteration.
+__device__ __forceinline__ void scale_acc(float& o, float f) {
+  float t;
+  asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\tv_accvgpr_write_b32 %0, %1"
+               : "+a"(o), "=&v"(t) : "v"(f));
+}
+
+// whole vectors in AGPRs here (vectors put together element by element would make the
+// compiler carry O through the loop as single registers)
+template <int N>
+__device__ __forceinline__ void hold_acc(f32x16 (&o)[N]) {
+#pragma unroll
+  for (int b = 0; b < N; ++b) asm volatile("" : "+a"(o[b]));
+}
+
+// Flash attention of one unit: four waves, one per SIMD (D = 256), each with 32 NB query
+// rows (tokens x heads of one KV head, GQA packed) over the unit's key tiles of 32.
+// Per wave and tile: S^T = K Q^T (v_mfma_f32_32x32x16_bf16 / _f16, Q^T operands in
+// registers), probabilities against a lazy reference max (fp32, log2 domain), O^T += V^T P^T
+// on v_mfma_f32_32x32x16_f16 (P and V in fp16, see kVShift), V^T by ds_read_b64_tr_b16.
+//
+// Bound by the matrix cores' power and by what a wave can issue beside its MFMAs.  NB = 2
+// needs 256 AGPRs (O) and all 256 VGPRs (Q^T 128, S 32, P 32, K operands two K-steps
+// ahead; a third one spills Q^T), so one wave per SIMD, and that wave has to overlap its
+// own MFMA and VALU work:
+//  - PV of tile t - 1 runs beside the softmax of tile t, whose maximum is not waited for:
+//    P is formed against the old reference, and only a row whose sum shows a large value
+//    has it redone;
+//  - an MFMA leaves room for about five other instructions (measured: 32.9 cycles with
+//    four, 44 with eight, 5 each beyond), so the rest is dealt out between the MFMAs;
+//  - the tile moves are LDS DMA (no registers, no ds_write), one beside every eighth
+//    MFMA: issued together they cost 900 cycles a tile, spread about 170;
+//  - rare blocks (mask, moved reference, ragged tiles) are marked unlikely, so that the
+//    loop is one run of code: in line they cost 800 of 3900 cycles a tile.
+// Per K/V operand read from LDS NB MFMAs run.  15360 + 9256 tokens, 6 heads: 3150 cycles
+// per 256 rows x 32 keys (2048 of MFMA) at the 1.9 GHz the power allows.  The call with
+// its other launches: 1900 us before (four waves of 32 rows, tiles through registers, one
+// phase after the other), 1230 us now, 0.92 PFLOP/s; a large library bf16 product reaches
+// 1.2 on this card.
+template <int D, int QT, int NB>
+__global__ __launch_bounds__(kThreads, prefill_wgs(D, NB)) void prefill_kernel(PrefillParams P) {
   using QV = typename QVec<QT>::type;    // one MFMA operand in the query dtype
   const oscar_prefill_args_v1& A = P.a;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int m = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5;
   const int G = P.group;
-  const int ntiles_q = (int)((A.num_tokens + P.qtok - 1) / P.qtok);
   const int kvh = blockIdx.y;
   const int64_t hist = A.history;
   const int64_t hk = A.num_kv_heads;
-  // this workgroup's unit: query tile qt over key tiles [kb, ke); slot >= 0: the tile
-  // is split and this unit writes a partial
-  int qt, kb = 0, slot = -1;
-  if (P.split) {
+  // this wave's query tile qt and the workgroup's key tiles [kb, ke); slot >= 0: the
+  // tile is split and this unit writes a partial.  NB == 2: waves 0-1 take the heavier
+  // tile of a pair, waves 2-3 the next one (live: it has this chunk).
+  int qt, kb = 0, ke, slot = -1;
+  bool live = true;
+  {
     const int u = blockIdx.x;
-    int c = 0;
+    int c = 0, idx;
+    if (P.split) {
+      const int* base = NB == 2 ? P.pbase : P.base;
 #pragma unroll
-    for (int cc = 1; cc < kMaxChunks; ++cc)
-      if (cc < P.chunks && u >= P.base[cc]) c = cc;
-    const int idx = u - P.base[c];
-    qt = ntiles_q - 1 - idx;  // heaviest (latest) query tiles first within a chunk class
-    kb = c * P.U;
-    if (qt >= P.qmin1) slot = c == 0 ? idx : u - P.qmin1;
-  } else {
-    qt = ntiles_q - 1 - (int)blockIdx.x;  // heaviest (latest) query tiles first
+      for (int cc = 1; cc < kMaxChunks; ++cc)
+        if (cc < P.chunks && u >= base[cc]) c = cc;
+      idx = NB * (u - base[c]);
+      kb = c * P.U;
+    } else {
+      idx = NB * u;
+    }
+    const int qt_top = P.ntq - 1 - idx;  // heaviest (latest) query tiles first within a chunk class
+    const int64_t q1_top = ((int64_t)qt_top + 1) * P.qtok;
+    ke = (int)tile_keys(hist, q1_top < A.num_tokens ? q1_top : A.num_tokens);
+    if (P.split && kb + P.U < ke) ke = kb + P.U;  // kb < ke (plan)
+    if (NB == 2 && wave >= 2) {
+      ++idx;
+      live = idx < (P.split ? P.base[c + 1] - P.base[c] : P.ntq);
+    }
+    qt = live ? P.ntq - 1 - idx : qt_top;
+    if (P.split && live && qt >= P.qmin1) slot = c == 0 ? idx : P.base[c] + idx - P.qmin1;
   }
   const int64_t q0 = (int64_t)qt * P.qtok;
   const int64_t q1 = (q0 + P.qtok < A.num_tokens) ? q0 + P.qtok : A.num_tokens;
-  const int64_t nkeys = hist + q1;  // keys visible to the last query of the tile
+  // this wave's own key tiles end at ke_own: the lighter tile of a pair may see fewer, and
+  // must not multiply values past them (0 x inf)
+  int ke_own = (int)tile_keys(hist, q1);
+  ke_own = !live || ke_own <= kb ? kb + 1 : ke_own < ke ? ke_own : ke;
 
-  // double-buffered key tiles.  K rows are padded by 16 bytes (row-per-lane 16-byte
-  // reads of 8 consecutive keys cover all banks), V rows by 32 bytes (the transpose
-  // reads of 4 consecutive keys x 32 bytes cover all banks)
-  __shared__ __attribute__((aligned(16))) uint16_t s_k[2][kKeys][D + 8];
-  __shared__ __attribute__((aligned(16))) uint16_t s_v[2][kKeys][D + 16];
-
-  // fill mapping: pass i, thread -> key i * KPP + tid / CPR, 16-byte column tid % CPR,
-  // so that a wave reads (and stores to LDS) whole contiguous key rows
-  constexpr int CPR = D / 8;              // 16-byte columns per key row
-  constexpr int KPP = kThreads / CPR;     // keys per pass
-  constexpr int NPASS = kKeys / KPP;
-  const int fkey = tid / CPR, fcol = tid % CPR;
-  u32x4 kr[NPASS], vr[NPASS];
-  bool vcur[NPASS];  // the V row is a current-chunk row (query dtype, not PV format)
-  // branch-free, 32-bit element offsets (the host checks they fit): keys past the
-  // chunk read current-chunk row 0, finite data whose scores the causal mask removes
-  const uint16_t* hk_base = P.hist_k + kvh * D + 8 * fcol;
-  const uint16_t* hv_base = P.hist_v + kvh * D + 8 * fcol;
-  const uint16_t* ck_base = (const uint16_t*)A.k + kvh * D + 8 * fcol;
-  const uint16_t* cv_base = (const uint16_t*)A.v + kvh * D + 8 * fcol;
-  const int hrow = (int)(hk * D), crow = (int)A.kv_stride_token;
-  const int ihist = (int)hist, ikeys = (int)nkeys;
-  auto fetch = [&](int kt) {
+  // Key tiles arrive by LDS DMA, 16 bytes a lane in lane order, so rows are not padded;
+  // the 16-byte columns of a row are permuted instead (each lane asks for the column that
+  // belongs at its place): K column c of key r at c ^ (r % 16), so that a row-per-lane
+  // read covers all banks; V column c at c ^ 4 (r % VSW), so that the transpose reads of
+  // 8 keys x 64 bytes do.  Three K tiles (t read, t + 1 and t + 2 in flight) and five V
+  // tiles (t - 2 still read by slower waves, t - 1 read, t being converted to the PV
+  // format, t + 1 and t + 2 in flight).
+  constexpr int CPR = D / 8;             // 16-byte columns per key row
+  constexpr int VSW = CPR / 4;           // 64-byte column groups per key row
+  constexpr int ROWB = 2 * D;            // bytes per key row
+  constexpr int TILEB = kKeys * ROWB;
+  constexpr int RPI = 64 / CPR;          // key rows per DMA instruction
+  constexpr int NDMA = kKeys / kWaves / RPI;  // DMA instructions per wave and tile
+  constexpr int NK = 3, NV = 5;
+  __shared__ __attribute__((aligned(1024))) uint8_t s_tiles[(NK + NV) * TILEB];
+  typedef __attribute__((address_space(3))) uint8_t lds_u8;
+  lds_u8* const lds = (lds_u8*)s_tiles;
+  const unsigned lds0 = (unsigned)(uintptr_t)lds;
+  const int hrow = (int)(hk * D * 2), crow = (int)(A.kv_stride_token * 2);  // bytes
+  const uint64_t hist_k = (uint64_t)P.hist_k + kvh * ROWB, hist_v = (uint64_t)P.hist_v + kvh * ROWB;
+  const uint64_t cur_k = (uint64_t)A.k + kvh * ROWB, cur_v = (uint64_t)A.v + kvh * ROWB;
+  const unsigned ulane = lane;
+  const int ihist = (int)hist, ikeys = (int)(hist + A.num_tokens);
+  // a value behind a register the compiler cannot see through: what is derived from it is
+  // computed where it is used instead of staying live across the loop, which has no
+  // registers to spare
+  auto fresh = [&](unsigned x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); return x; };
+  // The DMAs of key tile kt: instruction i brings the key row r0 + RPI i of each lane.
+  // Keys past the chunk read current-chunk row 0, finite data whose scores the causal mask
+  // removes.  load_tile takes any tile; load_part is instruction i (K for i < NDMA, then
+  // V) of a tile that lies within the history or within the chunk (a Tile).
+  auto row0 = [&]() __attribute__((always_inline)) { return wave * (kKeys / kWaves) + fresh(ulane) / CPR; };
+  const unsigned kcol = ((ulane % CPR) ^ (row0() & 15)) * 16, vcol = ((ulane % CPR) ^ (4 * (row0() % VSW))) * 16;
+  auto load_tile = [&](int kt, unsigned kdst, unsigned vdst) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NPASS; ++i) {
-      const int p = kt * kKeys + i * KPP + fkey;
+    for (int i = 0; i < NDMA; ++i) {
+      const int p = kt * kKeys + (int)row0() + RPI * i;
       const bool in_hist = p < ihist;
-      const int ci = (in_hist || p >= ikeys) ? 0 : p - ihist;  // current-chunk index
-      const uint16_t* ks = in_hist ? hk_base + (unsigned)(p * hrow) : ck_base + (unsigned)(ci * crow);
-      const uint16_t* vs = in_hist ? hv_base + (unsigned)(p * hrow) : cv_base + (unsigned)(ci * crow);
-      kr[i] = *(const u32x4*)ks;
-      vr[i] = *(const u32x4*)vs;
-      vcur[i] = !in_hist;
+      const int ci = p < ikeys ? p - ihist : 0;  // current-chunk index
+      const uint64_t off = (uint64_t)(unsigned)(in_hist ? p : ci) * (unsigned)(in_hist ? hrow : crow);
+      const unsigned lo = (wave * (kKeys / kWaves) + RPI * i) * ROWB;
+      dma16(lds0 + kdst + lo, (const void*)((in_hist ? hist_k : cur_k) + off + (kcol ^ (unsigned)(RPI * i * 16))));
+      dma16(lds0 + vdst + lo, (const void*)((in_hist ? hist_v : cur_v) + off + (vcol ^ (unsigned)(4 * (RPI * i % VSW) * 16))));
     }
   };
-  auto stash = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < NPASS; ++i) {
-      *(u32x4*)&s_k[buf][i * KPP + fkey][8 * fcol] = kr[i];
-      u32x4 w = vr[i];
-      if constexpr (QT == OSCAR_BF16) {
-        if (vcur[i]) {  // bf16 current-chunk values to the PV format
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            w[e] = pv_bits<QT>(__uint_as_float(vr[i][e] << 16)) | (pv_bits<QT>(__uint_as_float(vr[i][e] & 0xffff0000u)) << 16);
-        }
-      }
-      *(u32x4*)&s_v[buf][i * KPP + fkey][8 * fcol] = w;
-    }
+  struct Tile {
+    uint64_t k, v;          // its first row
+    unsigned pitch;         // bytes
+    unsigned row;           // per lane: offset of row r0
+    unsigned kdst, vdst;    // where it goes in LDS, this wave's part
   };
+  auto whole = [&](int kt) __attribute__((always_inline)) {
+    const int p0 = kt * kKeys;
+    return p0 + kKeys <= ihist || (p0 >= ihist && p0 + kKeys <= ikeys);
+  };
+  auto tile_at = [&](int kt, unsigned kdst, unsigned vdst) __attribute__((always_inline)) {
+    const int p0 = kt * kKeys;
+    const bool in_hist = p0 < ihist;
+    Tile t;
+    t.pitch = (unsigned)(in_hist ? hrow : crow);
+    const uint64_t off = (uint64_t)(unsigned)(in_hist ? p0 : p0 - ihist) * t.pitch;
+    t.k = (in_hist ? hist_k : cur_k) + off;
+    t.v = (in_hist ? hist_v : cur_v) + off;
+    t.row = row0() * t.pitch;
+    t.kdst = lds0 + kdst + wave * (kKeys / kWaves) * ROWB;
+    t.vdst = lds0 + vdst + wave * (kKeys / kWaves) * ROWB;
+    return t;
+  };
+  auto load_part = [&](const Tile& t, int i) __attribute__((always_inline)) {
+    const bool v = i >= NDMA;
+    i = v ? i - NDMA : i;
+    const unsigned sw = (unsigned)((v ? 4 * (RPI * i % VSW) : RPI * i) * 16);
+    dma16((v ? t.vdst : t.kdst) + RPI * i * ROWB, (v ? t.v : t.k) + (uint64_t)(RPI * i) * t.pitch,
+          t.row + ((v ? vcol : kcol) ^ sw));
+  };
+  // bf16 current-chunk rows of a landed V tile to the PV format, in place (kVShift):
+  // 16-byte part i of this thread's share
+  constexpr int NCONV = TILEB / 16 / kThreads;
+  constexpr int CONVROWS = kThreads * 16 / ROWB;  // key rows of one part, over the workgroup
+  auto conv_at = [&](unsigned off, int i) __attribute__((always_inline)) {
+    return (__attribute__((address_space(3))) u32x4*)(lds + off + (wave * 64 + fresh(ulane)) * 16 + i * kThreads * 16);
+  };
+  auto conv_keep = [&](int kt, int i) __attribute__((always_inline)) {
+    // the history rows of a mixed tile are in the format
+    return (int)((wave * 64 + fresh(ulane)) * 16 / ROWB) < ihist - kt * kKeys - CONVROWS * i;
+  };
+  auto converts = [&](int kt) __attribute__((always_inline)) { return QT == OSCAR_BF16 && kt * kKeys + kKeys > ihist; };
+  auto k_tile = [&](int i) __attribute__((always_inline)) { return (unsigned)(i * TILEB); };
+  auto v_tile = [&](int i) __attribute__((always_inline)) { return (unsigned)((NK + i) * TILEB); };
+  auto next = [](int i, int ring) { return i + 1 == ring ? 0 : i + 1; };
 
-  const int kt_all = (int)tile_keys(hist, q1);
-  const int ke = (P.split && kb + P.U < kt_all) ? kb + P.U : kt_all;  // kb < kt_all (plan)
-  fetch(kb);
+  // in the order the loop waits for them
+  load_tile(kb, k_tile(0), v_tile(0));
+  load_tile(kb + 1, k_tile(1), v_tile(1));
 
-  // this lane's row
-  const int n = wave * 32 + m;
-  const int64_t qi = q0 + n / G;
-  const bool row_ok = (n < P.qtok * G) && (qi < q1);
-  const int head = kvh * G + n % G;
-  const uint16_t* qrow = (const uint16_t*)A.q + (row_ok ? qi : 0) * A.q_stride_token + (int64_t)head * D;
+  // this lane's row of a row block: row n of the query tile, query qi; computed again where
+  // it is needed
+  struct Row { int n, head; int64_t qi; bool ok; };
+  auto row_of = [&](int nb) __attribute__((always_inline)) {
+    const int rm = (int)(fresh(ulane) & 31);
+    Row r;
+    r.n = NB == 2 ? (wave & 1) * 64 + 32 * nb + rm : wave * 32 + rm;
+    r.qi = q0 + r.n / G;
+    r.head = kvh * G + r.n % G;
+    r.ok = live && (r.n < P.qtok * G) && (r.qi < q1);
+    return r;
+  };
   // the wave's Q^T operands (K-step j) in registers for the whole key range: each
   // tile's QK then reads only K from LDS
-  QV qreg[D / 16];
+  QV qreg[NB][D / 16];
 #pragma unroll
-  for (int j = 0; j < D / 16; ++j)
-    qreg[j] = __builtin_bit_cast(QV, row_ok ? *(const u32x4*)(qrow + 16 * j + 8 * g) : u32x4{0u, 0u, 0u, 0u});
+  for (int nb = 0; nb < NB; ++nb) {
+    const Row r = row_of(nb);
+    const uint16_t* qrow = (const uint16_t*)A.q + (r.ok ? r.qi : 0) * A.q_stride_token + (int64_t)r.head * D;
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j)
+      qreg[nb][j] = __builtin_bit_cast(QV, r.ok ? *(const u32x4*)(qrow + 16 * j + 8 * g) : u32x4{0u, 0u, 0u, 0u});
+  }
   const float c = A.scale * kLog2e;
-  const int64_t limit = hist + qi + 1;  // keys [0, limit) visible to this row
 
-  float m_run = -INFINITY, l_run = 0.f;
-  f32x16 O[D / 32];
+  float m_run[NB], l_run[NB];
+  f32x16 O[NB][D / 32];
 #pragma unroll
-  for (int b = 0; b < D / 32; ++b)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) O[b][r] = 0.f;
-
-  stash(kb & 1);
-  if (kb + 1 < ke) fetch(kb + 1);
-  __syncthreads();
-  // The tile loop does no VALU work on O (kept in AGPRs by the MFMAs): a tile whose
-  // row max drifts more than kLazy above the reference leaves the loop, O and l are
-  // rescaled once, and the loop resumes at that tile (its QK is recomputed).
-  int kt = kb;
-  float m_move = -INFINITY;  // per row: the max that forced the exit
-  while (true) {
-    for (; kt < ke; ++kt) {
-      const int buf = kt & 1;
-      const int64_t k0 = (int64_t)kt * kKeys;
-      // ---- S^T = K Q^T; the operands of kQK K-steps are read from LDS together so
-      // that one LDS latency covers kQK MFMAs
-      f32x16 S = {};
-#pragma unroll
-      for (int j0 = 0; j0 < D / 16; j0 += kQK) {
-        QV ka[kQK], qa[kQK];
-#pragma unroll
-        for (int j = 0; j < kQK; ++j) {
-          ka[j] = *(const QV*)&s_k[buf][m][16 * (j0 + j) + 8 * g];
-          qa[j] = qreg[j0 + j];
-        }
-#pragma unroll
-        for (int j = 0; j < kQK; ++j) {
-          if constexpr (QT == OSCAR_F16) S = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[j], qa[j], S, 0, 0, 0);
-          else S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[j], qa[j], S, 0, 0, 0);
-        }
-        // keep the group's LDS reads ahead of its MFMAs (one latency per group)
-        __builtin_amdgcn_sched_group_barrier(0x100, kQK, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, kQK, 0);
-      }
-      const bool full = (k0 + kKeys <= hist + q0 + 1);  // visible to every row of the tile
-      // masked keys get -inf scores (boundary tiles only).  Padding rows have zero
-      // queries and are never written, so they need no mask.
-      if (!full) {
-        const int lim = (int)(limit - k0);  // keys of the tile visible to this row
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int pk = 8 * (r >> 2) + 4 * g + (r & 3);
-          S[r] = pk >= lim ? -INFINITY : S[r];
-        }
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[r]);
-      {
-        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-        mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c;  // c > 0
-      }
-      // a row's first visible key sets its reference (O and l are still zero there)
-      if (m_run == -INFINITY) m_run = mx;
-      if (__any(mx > m_run + kLazy)) {
-        m_move = mx;
-        break;
-      }
-      // p = 2^(S c - m) (exp2 of -inf is 0); rows with no key yet keep m = -inf and p = 0
-      const float nm = (m_run == -INFINITY) ? 0.f : -m_run;
-      // P in fp16 (p <= 2^kLazy; relative error 2^-12 per element)
-      f16x8 pb[2];
-      float lsum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; r += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(S[r], c, nm));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(S[r + 1], c, nm));
-        lsum += p0 + p1;
-        const f16x2 h = __builtin_convertvector(f32x2{p0, p1}, f16x2);
-        pb[r >> 3][r & 7] = h[0];
-        pb[r >> 3][(r & 7) + 1] = h[1];
-      }
-      l_run += lsum;
-      // ---- O^T += V^T P^T; the V^T operands of two output blocks (8 transpose reads)
-      // are read together
-      const int G16 = lane >> 4, i16 = lane & 15;
-#pragma unroll
-      for (int b0 = 0; b0 < D / 32; b0 += 2) {
-        f16x8 va[2][2];
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-          for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const int key = 16 * s + 4 * (G16 >> 1) + 8 * h + (i16 >> 2);
-              const uint16_t* addr = &s_v[buf][key][32 * (b0 + bb) + 16 * (G16 & 1) + 4 * (i16 & 3)];
-              auto t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(addr));
-#pragma unroll
-              for (int e = 0; e < 4; ++e) va[bb][s][4 * h + e] = __builtin_bit_cast(_Float16, (unsigned short)t[e]);
-            }
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-          for (int s = 0; s < 2; ++s)
-            O[b0 + bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[bb][s], pb[s], O[b0 + bb], 0, 0, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 1);
-      }
-      // the prefetched tile kt+1 goes to the other buffer (last read before the previous
-      // barrier), then tile kt+2 is prefetched; one barrier per tile
-      if (kt + 1 < ke) {
-        stash(buf ^ 1);
-        if (kt + 2 < ke) fetch(kt + 2);
-      }
-      __syncthreads();
-    }
-    if (kt >= ke) break;
-    // rare: rescale to the new reference and redo tile kt (its buffers are intact)
-    const bool move = m_move > m_run + kLazy;
-    const float f = move ? exp2f(m_run - m_move) : 1.f;
+  for (int nb = 0; nb < NB; ++nb) {
+    m_run[nb] = -INFINITY;
+    l_run[nb] = 0.f;
 #pragma unroll
     for (int b = 0; b < D / 32; ++b)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) O[b][r] *= f;
-    l_run *= f;
-    if (move) m_run = m_move;
+      for (int r = 0; r < 16; ++r) O[nb][b][r] = 0.f;
+    hold_acc(O[nb]);
   }
+
+  f32x16 S[NB];
+  u32x4 p_cur[NB][2], p_new[NB][2] = {};  // P^T of the tile before and of this one, fp16
+  float lsum[NB];
+
+  // ---- operands from a tile in LDS: K of K-step j; V of PV step i (output block i / 2, 16
+  // keys i % 2).  KA / VA of them are read ahead of their MFMAs, the first ones before
+  // the phase starts.
+  constexpr int KA = NB == 2 ? 3 : 4, VA = 3;
+  QV ka[KA];
+  f16x8 va[VA];
+  const unsigned krow = (ulane & 31) * ROWB, ksw = ((ulane >> 5) ^ (ulane & 15)) * 16;
+  auto k_op = [&](unsigned off, int j) __attribute__((always_inline)) {
+    return *(const __attribute__((address_space(3))) QV*)(lds + off + krow + (fresh(ksw) ^ (unsigned)(32 * j)));
+  };
+  const unsigned vkey = 4 * (ulane >> 5) + ((ulane & 15) >> 2);  // + 16 s + 8 h
+  const unsigned vrow = vkey * ROWB + 32 * ((ulane >> 4) & 1) + 8 * (ulane & 3), vsw = 64 * (vkey % VSW);
+  auto v_op = [&](unsigned off, int i) __attribute__((always_inline)) {
+    const lds_u8* const at = lds + off + vrow + ((unsigned)(64 * (i >> 1)) ^ fresh(vsw)) + 16 * (i & 1) * ROWB;
+    f16x8 v;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      auto t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(at + 8 * h * ROWB));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * h + e] = __builtin_bit_cast(_Float16, (unsigned short)t[e]);
+    }
+    return v;
+  };
+  auto k_ahead = [&](unsigned off) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < KA - 1; ++j) ka[j] = k_op(off, j);
+  };
+  auto v_ahead = [&](unsigned off) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < VA - 1; ++i) va[i] = v_op(off, i);
+  };
+  // ---- S^T = K Q^T of the landed tile kt, whose first K operands are in ka; reads the
+  // first V operands of the tile at `voff`, which PV takes next.
+  // An MFMA takes 32 cycles of the wave's SIMD, in which the wave can issue about five
+  // other instructions; more than that wait for nothing to overlap with.  The work that
+  // is not PV's is therefore dealt out one piece per MFMA: the DMAs of tile `t` (LOAD),
+  // the move of the last P to p_cur and the conversion of kt's V (CONV).
+  auto qk = [&](int kt, unsigned off, unsigned voff, unsigned vconv, const Tile& t, auto conv, auto load) __attribute__((always_inline)) {
+    constexpr bool CONV = decltype(conv)::value, LOAD = decltype(load)::value;
+    constexpr int NS = D / 16;
+    constexpr int MOVES = (8 * NB + NS - 1) / NS;  // per step, of the 8 NB registers of P
+    u32x4 cx;
+    bool keep = false;
+    auto beside = [&](int j, int nb) __attribute__((always_inline)) {
+      const int w = NB * j + nb;  // the MFMA of row block nb of K-step j
+      if (nb == 0 && j + KA - 1 < NS) ka[(j + KA - 1) % KA] = k_op(off, j + KA - 1);
+      if (nb == 0 && j == NS - 2) v_ahead(voff);
+      if (LOAD && w % (NB * NS / (2 * NDMA)) == 0) load_part(t, w / (NB * NS / (2 * NDMA)));
+      if constexpr (CONV) {
+        constexpr int WPC = NB * NS / NCONV;  // MFMAs per 16-byte part
+        const int i = w / WPC, q = w % WPC;
+        if (q == 0) cx = *conv_at(vconv, i);
+        if (q == WPC / 2) keep = conv_keep(kt, i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (q == WPC / 2 + e * (WPC / 2) / 4) {
+            const unsigned w = pv_pair(cx[e]);
+            cx[e] = keep ? cx[e] : w;
+          }
+        if (q == WPC - 1) *conv_at(vconv, i) = cx;
+      }
+      if (nb == NB - 1) {
+#pragma unroll
+        for (int e = MOVES * j; e < MOVES * (j + 1) && e < 8 * NB; ++e) {
+          unsigned x;
+          asm volatile("v_mov_b32 %0, %1" : "=v"(x) : "v"(p_new[e / 8][e / 4 % 2][e % 4]));
+          p_cur[e / 8][e / 4 % 2][e % 4] = x;
+        }
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        if (j == 0) mfma_qk<QT, true>(S[nb], ka[j % KA], qreg[nb][j]);
+        else mfma_qk<QT, false>(S[nb], ka[j % KA], qreg[nb][j]);
+        beside(j, nb);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // the MFMAs' results are read by the VALU next
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) asm volatile("s_nop 15" : "+v"(S[nb]));
+  };
+  // masked keys get -inf scores (boundary tiles only).  Padding rows have zero queries
+  // and are never written, so they need no mask.
+  const int all_see = (int)(hist + q0 + 1);  // keys visible to every row of the wave's tile
+  auto mask = [&](int kt) __attribute__((always_inline)) {
+    const int k0 = kt * kKeys;
+    if (__builtin_expect(k0 + kKeys <= all_see, 1)) return;
+    const int ml = (int)(fresh(ulane) >> 5);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int lim = (int)(hist + row_of(nb).qi + 1) - k0 - 4 * ml;  // keys of the tile visible to this row
+#pragma unroll
+      for (int r = 0; r < 16; ++r) S[nb][r] = 8 * (r >> 2) + (r & 3) >= lim ? -INFINITY : S[nb][r];
+    }
+  };
+  // p = 2^(S c - m) of element r (exp2 of -inf is 0; rows with no key yet have m = -inf and p = 0)
+  auto prob = [&](int nb, int r, float nm) __attribute__((always_inline)) { return __builtin_amdgcn_exp2f(fmaf(S[nb][r], c, nm)); };
+  auto neg_m = [&](int nb) __attribute__((always_inline)) { return m_run[nb] == -INFINITY ? 0.f : -m_run[nb]; };
+  auto row_max = [&](int nb) __attribute__((always_inline)) {  // of the scores, over both halves of the row
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[nb][r]);
+    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c;  // c > 0
+  };
+  auto put_p = [&](int nb, int r, float p0, float p1) __attribute__((always_inline)) {
+    unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{p0, p1}, f16x2));
+    asm volatile("" : "+v"(w));  // stays where it stands (else it sinks past the test for a moved reference)
+    p_new[nb][r >> 3][(r & 7) >> 1] = w;
+  };
+  // the probabilities of S against the reference m_run, not beside anything (first tile,
+  // moved reference)
+  auto softmax = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const float nm = neg_m(nb);
+      lsum[nb] = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        const float p0 = prob(nb, r, nm), p1 = prob(nb, r + 1, nm);
+        lsum[nb] += p0 + p1;
+        put_p(nb, r, p0, p1);
+      }
+    }
+  };
+  // ---- O^T += V^T P^T of the tile before, whose first V operands are in va, beside the
+  // probabilities and row sums of this tile (SM); reads the first K operands of the tile
+  // at `koff`
+  auto pv = [&](unsigned off, unsigned koff, auto sm) __attribute__((always_inline)) {
+    constexpr bool SM = decltype(sm)::value;
+    constexpr int NPV = D / 16;   // steps
+    constexpr int EPS = 16 / NPV; // elements of S per row block and step
+    float nm[NB], pe[NB][2];
+    if constexpr (SM) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) { nm[nb] = neg_m(nb); lsum[nb] = 0.f; }
+    }
+    auto pair_done = [&](int nb, int r) __attribute__((always_inline)) {  // elements r - 1, r
+      lsum[nb] += pe[nb][0] + pe[nb][1];
+      put_p(nb, r - 1, pe[nb][0], pe[nb][1]);
+    };
+#pragma unroll
+    for (int i = 0; i < NPV; ++i) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        O[nb][i >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[i % VA], __builtin_bit_cast(f16x8, p_cur[nb][i & 1]), O[nb][i >> 1], 0, 0, 0);
+        if (nb == 0 && i + VA - 1 < NPV) va[(i + VA - 1) % VA] = v_op(off, i + VA - 1);
+        if (SM && nb == NB - 1 && i == NPV - 1) k_ahead(koff);
+        if constexpr (SM) {
+          // a pair's sum and packing beside the next step's element
+#pragma unroll
+          for (int e = 0; e < EPS; ++e) {
+            const int r = EPS * i + e;
+            if (r % 2 == 0 && r > 0) pair_done(nb, r - 1);
+            pe[nb][r & 1] = prob(nb, r, nm[nb]);
+            if (r == 15) pair_done(nb, r);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // ---- the first tile: its row maxima are the first references
+  tile_barrier<2 * NDMA>();
+  load_tile(kb + 2, k_tile(2), v_tile(2));
+  k_ahead(k_tile(0));
+  qk(kb, k_tile(0), v_tile(0), v_tile(0), Tile{}, std::integral_constant<bool, QT == OSCAR_BF16>{}, std::false_type{});
+  mask(kb);
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) m_run[nb] = row_max(nb);
+  softmax();
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) l_run[nb] = lsum[nb];
+  tile_barrier<2 * NDMA>();  // as in the loop
+  k_ahead(k_tile(1));
+  // Iteration kt: QK of kt, then PV of kt - 1 beside the softmax of kt against the
+  // reference as it stands.  A row whose probabilities turn out large (one above 2^kLazy
+  // shows in their sum) or that had no visible key before moves its reference to its
+  // maximum: O and l are rescaled and P is formed again (rare).
+  int kr = 0, vr = 0;  // ring places of K(kt - 1) and V(kt - 1)
+#pragma clang loop unroll(disable)
+  for (int kt = kb + 1; kt < ke_own; ++kt) {
+    const int k1 = next(kr, NK), v1 = next(vr, NV);
+    // kt + 2 (past the last tile: that one again, never read) goes over K(kt - 1) and
+    // V(kt - 3), read before the last barrier
+    const int kn = kt + 2 < ke ? kt + 2 : ke - 1;
+    const unsigned kdst = k_tile(kr), vdst = v_tile(vr < 2 ? vr + NV - 2 : vr - 2);
+    if (__builtin_expect(!whole(kn), 0)) {
+      load_tile(kn, kdst, vdst);
+      qk(kt, k_tile(k1), v_tile(vr), v_tile(v1), Tile{}, std::integral_constant<bool, QT == OSCAR_BF16>{}, std::false_type{});
+    } else if (converts(kt)) {
+      qk(kt, k_tile(k1), v_tile(vr), v_tile(v1), tile_at(kn, kdst, vdst), std::true_type{}, std::true_type{});
+    } else {
+      qk(kt, k_tile(k1), v_tile(vr), v_tile(v1), tile_at(kn, kdst, vdst), std::false_type{}, std::true_type{});
+    }
+    // every wave is past QK of kt and PV of kt - 2; kt's V is in its format; kt + 1 has
+    // landed (kt + 2's DMAs are outstanding)
+    tile_barrier<2 * NDMA>();
+    mask(kt);
+    pv(v_tile(vr), k_tile(next(k1, NK)), std::true_type{});
+    kr = k1;
+    vr = v1;
+    bool moved = false;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) moved = moved || lsum[nb] > (float)(1 << kLazy) || m_run[nb] == -INFINITY;
+    if (__builtin_expect(__any(moved), 0)) {
+      asm volatile("s_nop 15\n\ts_nop 15");  // the PV MFMAs' results
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const float mx = row_max(nb);
+        const bool move = mx > m_run[nb];
+        const float f = move ? exp2f(m_run[nb] - mx) : 1.f;
+#pragma unroll
+        for (int b = 0; b < D / 32; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            float o = O[nb][b][r];
+            scale_acc(o, f);
+            O[nb][b][r] = o;
+          }
+        hold_acc(O[nb]);
+        l_run[nb] *= f;
+        if (move) m_run[nb] = mx;
+      }
+      softmax();
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) l_run[nb] += lsum[nb];
+  }
+  // the last tile (its V was converted before the last barrier)
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) { p_cur[nb][0] = p_new[nb][0]; p_cur[nb][1] = p_new[nb][1]; }
+  v_ahead(v_tile(vr));
+  pv(v_tile(vr), 0, std::false_type{});
+  // the other waves' tiles past this wave's own: its share of the moves and conversions
+#pragma clang loop unroll(disable)
+  for (int kt = ke_own; kt < ke; ++kt) {
+    const int v1 = next(vr, NV), kn = kt + 2 < ke ? kt + 2 : ke - 1;
+    load_tile(kn, k_tile(kr), v_tile(vr < 2 ? vr + NV - 2 : vr - 2));
+    if (converts(kt)) {
+      for (int i = 0; i < NCONV; ++i) {
+        u32x4 x = *conv_at(v_tile(v1), i);
+        const bool keep = conv_keep(kt, i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const unsigned w = pv_pair(x[e]);
+          x[e] = keep ? x[e] : w;
+        }
+        *conv_at(v_tile(v1), i) = x;
+      }
+    }
+    tile_barrier<2 * NDMA>();
+    kr = next(kr, NK);
+    vr = v1;
+  }
+  tile_barrier<0>();  // no DMA may be in flight when the workgroup ends
+
   // ---- finalize: row n = lane's row; O^T block b register r holds d = 32b + out_row(r, g)
-  float l_tot;
-  {
-    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
-    l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-  }
-  if (!row_ok) return;
-  // O back from the PV scale of bf16 V values (a power of two: exact)
-  const float inv = (l_tot > 0.f) ? (QT == OSCAR_F16 ? 1.f : (float)(1 << kVShift)) / l_tot : 0.f;
-  if (slot >= 0) {
-    // a chunk of a split tile: normalised O and its log2-domain LSE (-inf: no key of
-    // the chunk visible to the row) for prefill_merge_kernel
-    const int64_t prow = ((int64_t)slot * hk + kvh) * kRows + n;
-    float* po = P.part_o + prow * D;
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    float l_tot;
+    {
+      auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run[nb]), __float_as_uint(l_run[nb]), false, false);
+      l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    }
+    const Row row = row_of(nb);
+    const int rg = (int)(fresh(ulane) >> 5);
+    if (!row.ok) continue;
+    // O back from the PV scale of bf16 V values (a power of two: exact)
+    const float inv = (l_tot > 0.f) ? (QT == OSCAR_F16 ? 1.f : (float)(1 << kVShift)) / l_tot : 0.f;
+    const float lse2 = (l_tot > 0.f) ? m_run[nb] + log2f(l_tot) : -INFINITY;
+    if (slot >= 0) {
+      // a chunk of a split tile: normalised O and its log2-domain LSE (-inf: no key of
+      // the chunk visible to the row) for prefill_merge_kernel
+      const int64_t prow = ((int64_t)slot * hk + kvh) * kRows + row.n;
+      float* po = P.part_o + prow * D;
+#pragma unroll
+      for (int b = 0; b < D / 32; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+          *(f32x4*)(po + 32 * b + 8 * (r >> 2) + 4 * rg) = f32x4{O[nb][b][r] * inv, O[nb][b][r + 1] * inv,
+                                                                O[nb][b][r + 2] * inv, O[nb][b][r + 3] * inv};
+      if (rg == 0) P.part_lse[prow] = lse2;
+      continue;
+    }
+    const int64_t obase = row.qi * A.out_stride_token + (int64_t)row.head * D;
 #pragma unroll
     for (int b = 0; b < D / 32; ++b)
 #pragma unroll
       for (int r = 0; r < 16; r += 4)
-        *(f32x4*)(po + 32 * b + 8 * (r >> 2) + 4 * g) =
-            f32x4{O[b][r] * inv, O[b][r + 1] * inv, O[b][r + 2] * inv, O[b][r + 3] * inv};
-    if (g == 0) P.part_lse[prow] = (l_tot > 0.f) ? m_run + log2f(l_tot) : -INFINITY;
-    return;
+        store_out<QT>(A, obase + 32 * b + 8 * (r >> 2) + 4 * rg,
+                      f32x4{O[nb][b][r] * inv, O[nb][b][r + 1] * inv, O[nb][b][r + 2] * inv, O[nb][b][r + 3] * inv});
+    if (A.lse != nullptr && rg == 0) A.lse[row.qi * A.num_q_heads + row.head] = l_tot > 0.f ? lse2 * kLn2 : -INFINITY;
   }
-  const int64_t obase = qi * A.out_stride_token + (int64_t)head * D;
-#pragma unroll
-  for (int b = 0; b < D / 32; ++b)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = 32 * b + 8 * (r >> 2) + 4 * g + (r & 3);
-      const float v = O[b][r] * inv;
-      if (hist == 0) ((uint16_t*)A.out)[obase + d] = (uint16_t)q_bits<QT>(v);
-      else ((float*)A.out)[obase + d] = v;
-    }
-  if (A.lse != nullptr && g == 0)
-    A.lse[qi * A.num_q_heads + head] = (l_tot > 0.f) ? (m_run + log2f(l_tot)) * kLn2 : -INFINITY;
 }
 
 // FP32 LSE merge of a split tile's chunk partials (slab_attention.py:341-356 applied
@@ -522,14 +836,27 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams P) {
   }
   const float inv = L > 0.f ? 1.f / L : 0.f;
   const int head = kvh * G + n % G;
-  const int64_t obase = qi * A.out_stride_token + (int64_t)head * D + 4 * dq;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (A.history == 0) ((uint16_t*)A.out)[obase + e] = (uint16_t)q_bits<QT>(acc[e] * inv);
-    else ((float*)A.out)[obase + e] = acc[e] * inv;
-  }
+  store_out<QT>(A, qi * A.out_stride_token + (int64_t)head * D + 4 * dq, acc * inv);
   if (A.lse != nullptr && dq == 0)
     A.lse[qi * A.num_q_heads + head] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
+}
+
+// Two query tiles per workgroup from this many units on.  Below it the chip is not full
+// with one tile each (2048 fresh tokens are 247 units), and a unit's latency counts: one
+// tile takes about two thirds of a pair's time per key tile.  Above it pairs halve the
+// operand reads per MFMA (15360 + 9256 tokens: 1.23 ms against 1.60 ms unpaired).  At head
+// dim 128 two unpaired workgroups fit a CU and overlap each other (8000 + 4000 tokens, 16
+// heads on 2: 374 us against 380 us paired), so there are no pairs there.
+constexpr int64_t kPairUnits = 512;
+template <int D, int QT>
+void launch_prefill(const PrefillParams& p, dim3 grid, bool pairs, hipStream_t s) {
+  if constexpr (D == 256) {
+    if (pairs) {
+      hipLaunchKernelGGL((prefill_kernel<D, QT, 2>), grid, dim3(kThreads), 0, s, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((prefill_kernel<D, QT, 1>), grid, dim3(kThreads), 0, s, p);
 }
 
 }  // namespace
@@ -632,13 +959,17 @@ extern "C" int oscar_attn_prefill_v1(const oscar_prefill_args_v1* args, void* st
     }
     OSCAR_CHECK_LAUNCH("history_bf16_kernel");
   }
-  dim3 grid((unsigned)(p.split ? sp.units : p.ntq), (unsigned)a.num_kv_heads);
+  const int units = p.split ? sp.units : p.ntq;
+  const bool pairs = D == 256 && units * a.num_kv_heads > kPairUnits;
+  for (int c = 0; c < p.chunks; ++c) p.pbase[c + 1] = p.pbase[c] + (sp.base[c + 1] - sp.base[c] + 1) / 2;
+  const int wgs = !pairs ? units : p.split ? p.pbase[p.chunks] : (p.ntq + 1) / 2;
+  const dim3 grid((unsigned)wgs, (unsigned)a.num_kv_heads);
   if (a.q_dtype == OSCAR_F16) {
-    if (D == 256) hipLaunchKernelGGL((prefill_kernel<256, OSCAR_F16>), grid, dim3(kThreads), 0, s, p);
-    else hipLaunchKernelGGL((prefill_kernel<128, OSCAR_F16>), grid, dim3(kThreads), 0, s, p);
+    if (D == 256) launch_prefill<256, OSCAR_F16>(p, grid, pairs, s);
+    else launch_prefill<128, OSCAR_F16>(p, grid, pairs, s);
   } else {
-    if (D == 256) hipLaunchKernelGGL((prefill_kernel<256, OSCAR_BF16>), grid, dim3(kThreads), 0, s, p);
-    else hipLaunchKernelGGL((prefill_kernel<128, OSCAR_BF16>), grid, dim3(kThreads), 0, s, p);
+    if (D == 256) launch_prefill<256, OSCAR_BF16>(p, grid, pairs, s);
+    else launch_prefill<128, OSCAR_BF16>(p, grid, pairs, s);
   }
   OSCAR_CHECK_LAUNCH("prefill_kernel");
   if (p.split) {

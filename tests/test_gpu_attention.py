@@ -336,6 +336,63 @@ def test_prefill_split_matches_unsplit_and_oracle(cuda, prefix, n, d, hk, group,
     assert d_out <= tol and d_lse <= 1e-4
 
 
+@pytest.mark.parametrize("prefix,n,d,hk,group,qdt", [
+    (0, 6001, 256, 1, 16, "bf16"),    # paired query tiles, odd count, a ragged last tile
+    (1037, 5003, 256, 1, 16, "bf16"), # paired, a key tile of history and chunk rows
+    (1037, 5003, 256, 1, 16, "f16"),
+    (513, 3001, 256, 7, 3, "bf16"),   # paired, the lighter tile ends key tiles before the other
+    (0, 257, 256, 3, 1, "bf16"),      # one tile per workgroup, 128 tokens a tile
+    (95, 33, 256, 1, 6, "bf16"),      # one or two key tiles of everything
+    (1037, 3003, 128, 2, 8, "bf16"), (0, 4001, 128, 2, 8, "f16"), (40, 1, 128, 1, 5, "f16")])
+@pytest.mark.parametrize("split", [True, False])
+def test_prefill_tile_edges_match_oracle(cuda, prefix, n, d, hk, group, qdt, split):
+    """One and two query tiles per workgroup at the edges of tiles, chunks and the
+    history, on rows around them against the float64 oracle; the other rows finite."""
+    from oscar_amd import ops
+
+    hq, qtok = hk * group, 128 // group
+    c = cases.make_case([prefix], [n], fresh=True, seed=prefix + n + d, hk=hk, group=group, d=d)
+    tdt = torch.float16 if qdt == "f16" else torch.bfloat16
+    kw = dict(head_dim=d, split=split)
+    if prefix:
+        kw.update(history=prefix, k_cache=torch.from_numpy(c["k8"]).view(torch.int8).cuda(),
+                  v_cache=torch.from_numpy(c["v8"]).view(torch.int8).cuda(),
+                  block_table_row=torch.from_numpy(c["bt"][0]).cuda(),
+                  stage=tuple(torch.from_numpy(a).cuda() for a in c["stage"]))
+    lse = torch.full((n, hq), 7.0, dtype=torch.float32, device="cuda")
+    out = ops.attention_prefill(dev(c["q"], tdt), dev(c["k"], tdt), dev(c["v"], tdt), c["scale"], lse=lse, **kw)
+    torch.cuda.synchronize()
+    tiles = -(-n // qtok)
+    picked = [0, tiles // 2, max(tiles - 2, 0), tiles - 1]
+    rows = sorted({min(max(r, 0), n - 1) for t in picked for r in (t * qtok - 1, t * qtok, t * qtok + qtok - 1)})
+    ref_o, ref_l = attention_ref(c["q"], c["k"], c["v"], c["k8"], c["v8"], c["bt"], c["qsl"], c["seqs"], c["scale"],
+                                 c["stage"] if prefix else None, q_dtype=qdt, rows=rows)
+    out, lse = out.float().cpu().numpy(), lse.cpu().numpy()
+    assert np.isfinite(out).all() and np.isfinite(lse).all()
+    # the output's own rounding (16 bits without a history) beside OUT_TOL
+    ulp = 0.0 if prefix else (2.0 ** -10 if qdt == "f16" else 2.0 ** -8)
+    excess = (np.abs(out[rows] - ref_o[rows]) - (OUT_TOL + ulp * np.abs(ref_o[rows]))).max()
+    d_lse = np.abs(lse[rows] - ref_l[rows]).max()
+    print(f"{prefix}+{n} d={d} {hk}x{group} {qdt} split={split}: max|dO| "
+          f"{np.abs(out[rows] - ref_o[rows]).max():.3e}, max|dLSE| {d_lse:.3e}", flush=True)
+    assert excess <= 0 and d_lse <= 1e-3
+
+
+def test_prefill_values_past_a_tile_do_not_reach_it(cuda):
+    """inf in the values of the last tokens: the rows of earlier query tiles, which do not
+    see them, stay as they are, also in the tile that shares a workgroup with the last."""
+    from oscar_amd import ops
+
+    n, group = 2600, 32  # 650 query tiles of 4 tokens: paired
+    q, k, v = (cases.bf16_normal((n, h, 256), 90 + h) for h in (group, 1, 1))
+    clean = ops.attention_prefill(dev(q), dev(k), dev(v), 1 / 16, head_dim=256)
+    v[2592:] = np.inf  # the last two query tiles, in one key tile of their own
+    got = ops.attention_prefill(dev(q), dev(k), dev(v), 1 / 16, head_dim=256)
+    torch.cuda.synchronize()
+    assert torch.equal(got[:2592], clean[:2592])
+    assert not torch.isfinite(got[2596:].float()).any()
+
+
 def test_prefill_fp16_queries(cuda):
     """fp16 q/k/v: the fresh-only prefill returns fp16 (original domain); the
     continuation rounds the history fp16(x) (oracle with q_dtype f16)."""
