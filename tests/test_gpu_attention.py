@@ -436,6 +436,35 @@ def test_rotate_matches_fp32_reference(cuda):
         assert err < 1e-4, err
 
 
+@pytest.mark.parametrize("rows,d,xdt,odt,stride", [
+    (2559, 256, torch.float32, torch.bfloat16, 256), (2560, 256, torch.float32, torch.bfloat16, 256),
+    (2561, 256, torch.float32, torch.float32, 264), (8193, 256, torch.float32, torch.float16, 256),
+    (5120, 256, torch.bfloat16, torch.bfloat16, 256), (16417, 256, torch.bfloat16, torch.float32, 512),
+    (5151, 256, torch.float16, torch.float16, 256), (5119, 128, torch.float32, torch.float32, 128),
+    (5120, 128, torch.float32, torch.bfloat16, 128), (20481, 128, torch.float16, torch.float32, 136)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_rotate_row_counts_match_float64(cuda, rows, d, xdt, odt, stride, transpose):
+    """Both rotation kernels around the size where the second takes over (2.5 MiB of x),
+    with ragged last tiles and padded rows, against float64: three-term bf16 products err
+    by at most 2^-16 |x| |R| (columns of a rotation have norm 1), and the output rounds
+    once.  The rows are bounded by their norms, element by element."""
+    from oscar_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(rows + d)
+    x = torch.randn(rows, stride, generator=gen, device="cuda").to(xdt)[:, :d]
+    r = torch.from_numpy(cases.qr_rotation(d, 83)).cuda()
+    out = torch.full((rows + 1, d), 3.0, dtype=odt, device="cuda")
+    ops.rotate(x, r, transpose=transpose, out_dtype=odt, out=out[:rows])
+    torch.cuda.synchronize()
+    ref = x.double() @ (r.t().contiguous() if transpose else r).double()
+    ulp = {torch.float32: 2.0 ** -23, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[odt]
+    bound = 2.0 ** -16 * x.double().norm(dim=1, keepdim=True) + ulp * ref.abs() + 2.0 ** -24
+    excess = ((out[:rows].double() - ref).abs() - bound).max().item()
+    print(f"rotate {rows}x{d} {xdt} -> {odt}: max error past the bound {excess:.2e}", flush=True)
+    assert excess <= 0
+    assert (out[rows] == 3.0).all()
+
+
 @pytest.mark.parametrize("d,hk,group,mode", [(256, 1, 6, "write"), (128, 2, 4, "write"), (256, 1, 6, "write_clip"),
                                              (128, 2, 4, "invalidate")])
 def test_decode_write_sees_the_window_as_the_store_leaves_it(cuda, d, hk, group, mode):
