@@ -1370,7 +1370,7 @@ int check_args(const oscar_attn_args_v1& a, const char* name) {
 // store enqueued once the decode's arguments have passed, deferred (its quantization in
 // the merge launch) when it is a small call.
 int launch_checked(const oscar_attn_args_v1& a, const char* name, void* partials, int64_t partial_bytes,
-                   hipStream_t s, const oscar_store_args_v1* store = nullptr) {
+                   hipStream_t s, const oscar_store_args_v1* store = nullptr, const MetaCopy* meta = nullptr) {
   const int64_t D = a.cache.head_dim;
   if (D != 128 && D != 256) return fail(-22, "%s: head_dim %lld unsupported", name, (long long)D);
   if (a.num_items <= 0 || a.num_groups <= 0) {
@@ -1395,7 +1395,7 @@ int launch_checked(const oscar_attn_args_v1& a, const char* name, void* partials
     if (store->cache.head_dim != D)
       return fail(-22, "%s: the store's head_dim %lld differs from the decode's", name,
                   (long long)store->cache.head_dim);
-    const int rc = store_launch(store, s, a.phases == 0, name, &sp);
+    const int rc = store_launch(store, s, a.phases == 0, name, &sp, meta);
     if (rc != 0) return rc;
   }
   return D == 256 ? launch_decode<256>(p, s, sp) : launch_decode<128>(p, s, sp);
@@ -1440,6 +1440,12 @@ extern "C" int oscar_attn_decode_v1(const oscar_attn_args_v1* args, void* stream
   if (!args) return fail(-22, "oscar_attn_decode_v1: null args");
   return launch_checked(*args, "oscar_attn_decode_v1", args->workspace, args->workspace_bytes,
                         (hipStream_t)stream);
+}
+
+int oscar::decode_write_launch(const oscar_store_args_v1& store, const oscar_attn_args_v1& attn, const MetaCopy* meta,
+                               void* stream) {
+  return launch_checked(attn, "oscar_decode_write_v1", attn.workspace, attn.workspace_bytes, (hipStream_t)stream,
+                        &store, meta);
 }
 
 extern "C" int oscar_decode_write_v1(const oscar_store_args_v1* store, const oscar_attn_args_v1* attn,

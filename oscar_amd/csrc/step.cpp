@@ -6,13 +6,14 @@
 // of the split-K decode, up to kMaxSplitRows).  Per call: classify the
 // batch from the host metadata, build the split-K plan (oscar_attn_plan_v1) straight
 // into a pinned ring slot next to the request table, one host-to-device copy of the
-// slot, then the store (or the query rotation), the split-K decode + merge and the
+// slot (by the store's launch for a small store), then the store (or the query rotation), the split-K decode + merge and the
 // inverse rotation, all through the public entry points, on the caller's stream (the
 // store and decode as oscar_decode_write_v1).
 #include <mutex>
 #include <vector>
 
 #include "common.h"
+#include "store_quant.h"
 
 namespace oscar {
 namespace {
@@ -203,7 +204,11 @@ extern "C" int oscar_decode_step_v1(oscar_context_v1* ctx, oscar_step_args_v1* a
                 (long long)L.total);
   }
   const int64_t used = o_items + (int64_t)plan.num_items * OSCAR_WORK_INTS * 4;
-  if (hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, s) != hipSuccess)
+  // a step of a small store (deferred: nothing in it reads the slot) carries the slot in the
+  // store's launch; others copy it
+  MetaCopy meta;
+  if (has_new && n <= kFusedTokens && plan.num_items > 0) meta = MetaCopy{host, dev, align_up(used, 16)};
+  else if (hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, s) != hipSuccess)
     return fail(-5, "oscar_decode_step_v1: metadata copy failed");
   ctx->used[slot] = true;
   const int32_t* d_qsl = (const int32_t*)dev;
@@ -295,7 +300,7 @@ extern "C" int oscar_decode_step_v1(oscar_context_v1* ctx, oscar_step_args_v1* a
     at.q_dtype = a.q_dtype;
     // with new tokens: the store and the decode in one call (a small store's
     // quantization and slot / window writes ride in the decode's merge launch)
-    rc = has_new ? oscar_decode_write_v1(&st, &at, stream) : oscar_attn_decode_v1(&at, stream);
+    rc = has_new ? decode_write_launch(st, at, &meta, stream) : oscar_attn_decode_v1(&at, stream);
   }
   if (rc == 0) {
     oscar_rotate_args_v1 ro{};

@@ -49,9 +49,24 @@ struct StoreParams {
   int32_t deferred;  // small calls of oscar_decode_write_v1: store_small_kernel rotates only
                      // (read-path copies, rotated K / V in y, pending tags); the merge launch
                      // of the decode quantizes (quant_deferred)
+  // small calls: meta_vecs 16-byte vectors that extra workgroups of the launch copy from
+  // pinned host memory to the device, for the launches behind it on the stream
+  const u32x4* meta_src;
+  u32x4* meta_dst;
+  int32_t meta_vecs;
   int32_t slots31;   // capacity < 2^31: slots split into block and offset by div_bs
   FastDiv div_hk, div_hq, div_bs, div_rows;  // num_kv_heads, num_q_heads, block_size, staging rows
 };
+
+// Integer arrays of a call (16-byte aligned, whole vectors) on their way from the pinned
+// host ring to the device.
+struct MetaCopy {
+  const void* src = nullptr;
+  void* dst = nullptr;
+  int64_t bytes = 0;
+};
+// calls of at most this many tokens take the one-launch store, which can carry a MetaCopy
+constexpr int64_t kFusedTokens = 64;
 
 // Owner tag of a seat that a deferred small call rewrites, from its rotation launch to
 // its quantization: it matches no block, so a reader in between (the decode of
@@ -339,6 +354,12 @@ __device__ void quant_vector(const StoreParams& p, int kind, int64_t t, int64_t 
 // p.deferred = 1: read-path copies, rotated K / V in p.y, pending tags), the
 // quantization being left to quant_deferred in the decode's merge launch.  *out
 // receives the parameters; returns 0, or the negative error.
-int store_launch(const oscar_store_args_v1* args, void* stream, bool defer, const char* fn, StoreParams* out);
+int store_launch(const oscar_store_args_v1* args, void* stream, bool defer, const char* fn, StoreParams* out,
+                 const MetaCopy* meta = nullptr);
+
+// oscar_decode_write_v1 whose integer arrays (attn and store point at their device copies)
+// are still on the host: `meta` rides on the store's launch (small stores; empty: nothing)
+int decode_write_launch(const oscar_store_args_v1& store, const oscar_attn_args_v1& attn, const MetaCopy* meta,
+                        void* stream);
 
 }  // namespace oscar

@@ -151,6 +151,56 @@ def test_native_decode_step_matches_general_path_and_oracle(cuda, mode):
     assert diff <= 2e-2
 
 
+@pytest.mark.parametrize("requests", [1, 21, 64, 65])
+def test_native_step_metadata_follows_every_call(cuda, requests):
+    """The step's plan and request table travel in the store's launch up to 64 tokens and in
+    a copy of their own beyond.  Back to back steps whose lengths change from call to call
+    (a stale or torn table shows) against the general path, bytes of the written slots
+    included."""
+    from oscar_amd.backend import OscarAttentionBackendImpl  # noqa: F401
+
+    dev = torch.device("cuda", 0)
+    d, hq, hk, bs = 256, 6, 1, 128
+    g = np.random.default_rng(requests)
+    prefixes = [int(x) for x in g.integers(40, 900, requests)]
+    c = cases.make_case(prefixes, [1] * requests, seed=requests)
+    table = torch.from_numpy(c["bt"]).to(dev)
+    tq, tk, tv = (torch.from_numpy(c[x]).to(dev).bfloat16().view(requests, -1) for x in "qkv")
+    results = []
+    for native in (True, False):
+        impl, layer = OscarAttentionBackendImplFactory(), _Layer()
+        eye = torch.eye(d, dtype=torch.float32, device=dev)
+        layer._oscar_rots = (eye, eye)
+        caches = [torch.from_numpy(c[x]).view(torch.int8).to(dev).clone() for x in ("k8", "v8")]
+        impl._set_caches(caches)
+        impl._ensure_staging(layer, caches)
+        for arena, x in zip((layer._oscar_stage_k, layer._oscar_stage_v, layer._oscar_slot_owner), c["stage"]):
+            arena.copy_(torch.from_numpy(x))
+        outs = []
+        for step in range(6):
+            lens = [p - step * (r % 3) for r, p in enumerate(prefixes)]  # read shorter histories
+            md = _MD()
+            md.num_actual_tokens = requests
+            md.slot_mapping = torch.tensor([int(c["bt"][r, n // bs]) * bs + n % bs for r, n in enumerate(lens)], device=dev)
+            md.query_start_loc_cpu = torch.arange(requests + 1, dtype=torch.int32)
+            md.seq_lens_list = [n + 1 for n in lens]
+            md.block_tables = table
+            out = torch.empty(requests, hq * d, dtype=torch.bfloat16, device=dev)
+            if native:
+                assert impl._native_step(layer, tq, tk, tv, caches, md, out)
+            else:
+                impl._run(layer, tq, tk, tv, caches, md, out, write=True)
+            outs.append(out)
+        torch.cuda.synchronize()
+        results.append((torch.stack(outs).float(), *caches, layer._oscar_slot_owner))
+    (o1, k1, v1, w1), (o2, k2, v2, w2) = results
+    assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(w1, w2)
+    # both paths round the output to bf16 once; sums may differ in order by one ulp of it
+    excess = ((o1 - o2).abs() - (2e-3 + 2.0 ** -7 * o2.abs())).max().item()
+    print(f"{requests} requests: native vs general past one ulp {excess:.2e}", flush=True)
+    assert excess <= 0
+
+
 def OscarAttentionBackendImplFactory():
     from oscar_amd.backend import OscarAttentionBackendImpl
 
