@@ -42,6 +42,10 @@ MAX_DECODE_ROWS = 32  # rows (query tokens x heads per KV head) of one decode MF
 # and shares it between query tiles but walks it serially per query tile (at 24576
 # history tokens: 24-156 us for chunks of 8-400 tokens against 1.1 ms).
 MAX_SPLIT_ROWS = 32 * 512
+# Calls of more new tokens than this are looked over for prompts before the native step's
+# arguments are built (about 30 us that a batch with a prompt throws away; decode and
+# verify steps are smaller)
+MANY_TOKENS = 128
 
 
 # ---------------------------------------------------------------- metadata
@@ -345,11 +349,13 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
         if not (query.is_contiguous() and output.is_contiguous()) or query.numel() // (hq * d) < n:
             return False
         has_new = key is not None
+        if has_new and n > MANY_TOKENS and self._has_prompt(md, qsl, seqs, n):
+            return False
         if has_new and self._oscar.window_enabled:
             self._ensure_staging(layer, kv_cache)
-        stream = torch.cuda.current_stream(query.device).cuda_stream
+        stream = ops._stream(query.device)
         scratch = ops.DeviceScratch.get(query.device, stream)
-        a = self._step_args(layer, query.device, query.dtype)
+        a = self._step_args(layer, query.device, query.dtype, scratch)
         if a is None:
             return False
         a.query, a.output, a.num_tokens = query.data_ptr(), output.data_ptr(), n
@@ -393,13 +399,27 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
             self._oscar_stats["kv_bytes_written"] += n * hk * 160
         return True
 
-    def _step_args(self, layer, device, dtype):
+    def _has_prompt(self, md, qsl, seqs, n) -> bool:
+        """The batch holds a history-free request or a chunk past MAX_SPLIT_ROWS, which the
+        native step leaves to the general path.  False as well for a batch that the native
+        step refuses: its checks come first, and it words the errors."""
+        table = _block_tables(md)
+        group, bs = self.num_heads // self.num_kv_heads, self.key_cache.shape[1]
+        if group > MAX_DECODE_ROWS or table.ndim != 2 or table.shape[0] < len(qsl) - 1 or table.shape[1] < 1:
+            return False
+        starts, found = [min(s, n) for s in qsl.tolist()], False
+        for a, b, seq in zip(starts, starts[1:], seqs.tolist()):
+            if b < a or seq < 0 or b > a and (seq < b - a or -(-(seq - (b - a)) // bs) > table.shape[1]):
+                return False
+            found = found or b > a and (seq == b - a or (b - a) * group > MAX_SPLIT_ROWS)
+        return found
+
+    def _step_args(self, layer, device, dtype, scratch):
         """The layer's step arguments that stay fixed from call to call (caches, window
         arena, rotations, settings, scratch), rebuilt only when one of them changes."""
         d, hk = self.head_size, self.num_kv_heads
         rk, rv = self._layer_rots(layer, device)
         stage = self._stage(layer)
-        scratch = ops.DeviceScratch.get(device)
         bs = self.key_cache.shape[1]
         seats = 0 if stage is None else stage[2].shape[0] * bs
         slot_claims, seat_claims = scratch.claims(self.key_cache.shape[0] * bs, seats)

@@ -281,3 +281,46 @@ def test_mixed_batch_routes_slice_consecutive_decodes_and_gather_otherwise():
     assert b3.short == [0, 2] and b3.fresh == [3]
     assert impl._decode_route(b3)["span"] == (0, 3, 0, 5)
     assert impl._decode_route(b3)["qsl"] == [0, 4, 4, 5]
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_prompts_are_found_before_the_native_step(seed):
+    """The early look for prompts sends a batch down the general path exactly where the
+    native step would hand it back (a fresh request or a chunk past MAX_SPLIT_ROWS) and
+    leaves every batch that the native step refuses to it."""
+    import torch
+    from types import SimpleNamespace
+    from oscar_amd import backend as B
+
+    r = np.random.default_rng(seed)
+    impl = B.OscarAttentionBackendImpl.__new__(B.OscarAttentionBackendImpl)
+    impl.num_kv_heads, impl.key_cache = 1, torch.empty(4, 128, 1, 1)
+    for _ in range(200):
+        impl.num_heads = int(r.choice([1, 6, 32, 40]))
+        n = int(r.integers(1, 6))
+        chunks = [int(x) for x in r.choice([0, 1, 4, 300, 3000, 20000], n)]
+        seqs = [c + int(r.choice([0, 0, 5, 900])) for c in chunks]
+        flaw = r.choice(["none"] * 5 + ["rows", "cols", "short", "order", "negative"])
+        qsl = [0] + np.cumsum(chunks).tolist()
+        table = torch.zeros(n, 400, dtype=torch.int32)
+        if flaw == "rows":
+            table = table[:n - 1]
+        if flaw == "cols":
+            table, seqs = table[:, :7], [s + 1000 for s in seqs]
+        if flaw == "short":
+            seqs[int(np.argmax(chunks))] = max(chunks) - 1
+        if flaw == "order":
+            qsl[n // 2 + 1:] = [-1] * (n - n // 2)
+        if flaw == "negative":
+            seqs[0] = -3
+        actual = max(qsl[-1], 0)
+        got = impl._has_prompt(SimpleNamespace(block_tables=table), torch.tensor(qsl), np.asarray(seqs), actual)
+        group = impl.num_heads
+        refused = group > B.MAX_DECODE_ROWS or table.shape[0] < n or any(
+            b < a or s < 0 or b > a and (s < b - a or -(-(s - (b - a)) // 128) > table.shape[1])
+            for a, b, s in zip(qsl, qsl[1:], seqs))
+        if refused:
+            assert not got
+        else:
+            batch = B._Batch.classify(qsl, seqs, actual, True, group)
+            assert got == bool(batch.fresh or batch.long)
