@@ -288,8 +288,7 @@ def test_prompts_are_found_before_the_native_step(seed):
     """The early look for prompts sends a batch down the general path exactly where the
     native step would hand it back (a fresh request or a chunk past MAX_SPLIT_ROWS) and
     leaves every batch that the native step refuses to it."""
-    import torch
-    from types import SimpleNamespace
+    import numpy as np
     from oscar_amd import backend as B
 
     r = np.random.default_rng(seed)
@@ -314,7 +313,7 @@ def test_prompts_are_found_before_the_native_step(seed):
         if flaw == "negative":
             seqs[0] = -3
         actual = max(qsl[-1], 0)
-        got = impl._has_prompt(SimpleNamespace(block_tables=table), torch.tensor(qsl), np.asarray(seqs), actual)
+        got = impl._has_prompt(NS(block_tables=table), torch.tensor(qsl), np.asarray(seqs), actual)
         group = impl.num_heads
         refused = group > B.MAX_DECODE_ROWS or table.shape[0] < n or any(
             b < a or s < 0 or b > a and (s < b - a or -(-(s - (b - a)) // 128) > table.shape[1])
