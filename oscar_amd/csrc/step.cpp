@@ -70,7 +70,8 @@ extern "C" int oscar_context_create_v1(int32_t device, oscar_context_v1** out) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) != hipSuccess) rc = fail(-5, "oscar_context_create_v1: device properties");
   else c->cu_count = prop.multiProcessorCount;
-  if (!rc && hipHostMalloc((void**)&c->host_ring, kRingSlots * kSlotBytes, hipHostMallocDefault) != hipSuccess)
+  // coherent: kernels read the slots, which the host writes again for later calls
+  if (!rc && hipHostMalloc((void**)&c->host_ring, kRingSlots * kSlotBytes, hipHostMallocCoherent) != hipSuccess)
     rc = fail(-12, "oscar_context_create_v1: pinned ring allocation failed");
   if (!rc && hipMalloc((void**)&c->dev_ring, kRingSlots * kSlotBytes) != hipSuccess)
     rc = fail(-12, "oscar_context_create_v1: device ring allocation failed");
