@@ -143,15 +143,21 @@ def transient_parts(impl, max_tokens: int, max_model_len: int = 0, max_seqs: int
     (calls of up to max_tokens), the native step's (rotated q/k/v, out_rot, LSE and the
     item partials), the general decode's item partials, and the continuation prefill's
     (the bf16 history of up to max_model_len tokens and the partials of its split over
-    max_tokens query tokens)."""
+    up to max_tokens query tokens: shorter calls can split further than the longest one, into
+    at most 512 chunks of work and one more per query tile of 128 rows)."""
     lib = _lib_sizes()
     hq, hk, d = impl.num_heads, impl.num_kv_heads, impl.head_size
     items = decode_items_bound(max_tokens, max_model_len, hk, hq // hk, max_seqs)
+    prefill = max(0, lib.oscar_prefill_workspace_bytes_v2(max(max_model_len, 0), max_tokens, hq, hk, d))
+    if prefill > 0:
+        tiles = -(-max_tokens // (128 // (hq // hk)))
+        history = lib.oscar_prefill_workspace_bytes_v1(max(max_model_len, 0), hk, d)
+        prefill = max(prefill, history + 256 + (512 + tiles * hk) * 128 * (d + 1) * 4)
     return {
         "store": lib.oscar_store_workspace_bytes_v1(max_tokens, hk, d),
         "step": lib.oscar_step_workspace_bytes_v1(max_tokens, hq, hk, d, items),
         "decode": items * 32 * (d + 1) * 4,
-        "prefill": max(0, lib.oscar_prefill_workspace_bytes_v2(max(max_model_len, 0), max_tokens, hq, hk, d)),
+        "prefill": prefill,
     }
 
 
