@@ -9,7 +9,7 @@ arithmetic runs in liboscar_amd.so:
          scatter with last-writer-wins, owner tags and FP32 window, plus the rotated
          q/k/v the read path needs;
 * read   ``ops.attention_decode`` (cached requests; chunks of more than 32 rows per KV
-         head as 32-row sub-requests of the plan, up to LONG_CHUNK),
+         head as 32-row sub-requests of the plan, up to MAX_SPLIT_ROWS),
          ``ops.attention_prefill`` (longer continuation chunks; history-free requests in
          the original domain), then the inverse rotation ``ops.rotate(out_rot, R_v^T)``.
 
@@ -37,30 +37,11 @@ from .rotation import get_layer_rotation
 
 MAX_DECODE_ROWS = 32  # rows (query tokens x heads per KV head) of one decode MFMA tile
 # A cached chunk of more rows per KV head runs through the split-K decode as
-# sub-requests of MAX_DECODE_ROWS rows, each of which decodes the request's whole history;
-# past this many rows always through the MFMA prefill, which decodes it once for all.
+# sub-requests of MAX_DECODE_ROWS rows (each streams the request's history once), up to
+# this many rows; longer chunks go to the MFMA prefill, which decodes the history once
+# and shares it between query tiles but walks it serially per query tile (at 24576
+# history tokens: 24-156 us for chunks of 8-400 tokens against 1.1 ms).
 MAX_SPLIT_ROWS = 32 * 512
-# Below that, work (new tokens x query heads x width, half as much again for each 16384
-# history tokens) from which the prefill is the faster one, its route through the general
-# path included.  Measured (us, split-K / prefill; 6 heads of 256 on 1 unless said): 800
-# tokens over 3000 154 / 129, over 24576 327 / 220; 1600 over 8000 375 / 193; 16 heads of 128
-# on 2, 1024 over 15000 418 / 205.  Beside 16 decodes the general path takes 200 at least:
-# 800 over 1000 202 / 204, over 15000 302 / 206; 600 over 6000 147 / 203.
-LONG_CHUNK = 3 << 19
-
-
-def _chunk_is_long(tokens, history, group, hk, d, fp16):
-    """Whether a cached chunk goes to the prefill (step.cpp holds the same rule).  A chunk
-    much longer than its history stays on the split-K decode below MAX_SPLIT_ROWS: that adds
-    its own keys with probabilities of 16 bits' precision, the prefill with 11 (error against
-    float64, 2000 tokens over 300: bf16 3.36e-3 on both, fp16 4.2e-4 / 4.7e-4; over 2000:
-    3.6e-3 / 3.4e-3 and 6.6e-4 / 4.7e-4).  The prefill takes histories of up to 2^31 values."""
-    if tokens * group > MAX_SPLIT_ROWS:
-        return True
-    return (tokens * group * hk * d * (32768 + history) > LONG_CHUNK * 32768
-            and history * (1 if fp16 else 16) >= tokens and (history + 64) * hk * d < 1 << 31)
-
-
 # Calls of more new tokens than this are looked over for prompts before the native step's
 # arguments are built (about 30 us that a batch with a prompt throws away; decode and
 # verify steps are smaller)
@@ -162,10 +143,10 @@ class _Batch:
     fresh: list = field(default_factory=list)   # no history: original-domain prefill
     short: list = field(default_factory=list)   # cached, split-K decode (sub-requests of
                                                 # <= 32 rows per KV head for longer chunks)
-    long: list = field(default_factory=list)    # long cached chunk (_chunk_is_long): prefill
+    long: list = field(default_factory=list)    # cached chunk of more than MAX_SPLIT_ROWS: prefill
 
     @classmethod
-    def classify(cls, qsl, seqs, actual, has_new, group, hk=1, d=256, fp16=False):
+    def classify(cls, qsl, seqs, actual, has_new, group):
         b = cls([min(s, actual) for s in qsl], list(seqs), actual)
         for i in range(len(b.qsl) - 1):
             n = b.qsl[i + 1] - b.qsl[i]
@@ -173,8 +154,7 @@ class _Batch:
                 continue
             if has_new and b.seqs[i] == n:
                 b.fresh.append(i)
-            elif group <= MAX_DECODE_ROWS and (
-                    not has_new or not _chunk_is_long(n, b.seqs[i] - n, group, hk, d, fp16)):
+            elif group <= MAX_DECODE_ROWS and (not has_new or n * group <= MAX_SPLIT_ROWS):
                 b.short.append(i)
             else:
                 b.long.append(i)
@@ -371,8 +351,7 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
         if not (query.is_contiguous() and output.is_contiguous()) or query.numel() // (hq * d) < n:
             return False
         has_new = key is not None
-        if has_new and n > MANY_TOKENS and self._has_prompt(md, qsl, seqs, n, query.dtype == torch.float16) \
-                and not torch.cuda.is_current_stream_capturing():
+        if has_new and n > MANY_TOKENS and self._has_prompt(md, qsl, seqs, n):
             return False
         if has_new and self._oscar.window_enabled:
             self._ensure_staging(layer, kv_cache)
@@ -422,9 +401,9 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
             self._oscar_stats["kv_bytes_written"] += n * hk * 160
         return True
 
-    def _has_prompt(self, md, qsl, seqs, n, fp16=False) -> bool:
-        """The batch holds a history-free request or a long cached chunk, which the native
-        step leaves to the general path.  False as well for a batch that the native
+    def _has_prompt(self, md, qsl, seqs, n) -> bool:
+        """The batch holds a history-free request or a chunk past MAX_SPLIT_ROWS, which the
+        native step leaves to the general path.  False as well for a batch that the native
         step refuses: its checks come first, and it words the errors."""
         table = _block_tables(md)
         group, bs = self.num_heads // self.num_kv_heads, self.key_cache.shape[1]
@@ -434,8 +413,7 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
         for a, b, seq in zip(starts, starts[1:], seqs.tolist()):
             if b < a or seq < 0 or b > a and (seq < b - a or -(-(seq - (b - a)) // bs) > table.shape[1]):
                 return False
-            found = found or b > a and (seq == b - a or _chunk_is_long(
-                b - a, seq - (b - a), group, self.num_kv_heads, self.head_size, fp16))
+            found = found or b > a and (seq == b - a or (b - a) * group > MAX_SPLIT_ROWS)
         return found
 
     def _step_args(self, layer, device, dtype, scratch):
@@ -497,7 +475,7 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
         if write and has_new and (q3.shape[0] < n_md or k3.shape[0] < n_md or v3.shape[0] < n_md):
             raise ValueError("query/key/value hold fewer rows than num_actual_tokens")
         qsl, seqs = metadata_batch_lists(md)
-        batch = _Batch.classify(qsl, seqs, actual, has_new, group, hk, d, query.dtype == torch.float16)
+        batch = _Batch.classify(qsl, seqs, actual, has_new, group)
         stage_mode = STAGE_NONE
         if write and has_new:
             if self._oscar.window_enabled:

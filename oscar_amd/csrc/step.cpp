@@ -3,7 +3,7 @@
 // Replaces the Python orchestration of oscar_ascend/backend.py:249-393 (forward ->
 // write + window -> _streaming_attention -> inverse rotation) for batches whose
 // requests all have history (chunks of more than 32 rows per KV head run as sub-requests
-// of the split-K decode, up to the prefill's line).  Per call: classify the
+// of the split-K decode, up to kMaxSplitRows).  Per call: classify the
 // batch from the host metadata, build the split-K plan (oscar_attn_plan_v1) straight
 // into a pinned ring slot next to the request table, one host-to-device copy of the
 // slot (by the store's launch for a small store), then the store (or the query rotation), the split-K decode + merge and the
@@ -19,15 +19,9 @@ namespace oscar {
 namespace {
 
 constexpr int kRingSlots = 32;
-// Cached chunks that the step leaves to the prefill path, which decodes the history once for
-// all of its query tiles: more rows per KV head than kMaxSplitRows, and those of prefill_chunk
-// (backend.py, _chunk_is_long: the same rule, with the figures).
+// longest current chunk (rows per KV head) of a request the step takes: more rows go to
+// the prefill path, which decodes the history once for all of its query tiles
 constexpr int64_t kMaxSplitRows = 32 * 512;
-constexpr int64_t kLongChunk = 3 << 19;
-bool prefill_chunk(int64_t tokens, int64_t history, int64_t hq, int64_t hk, int64_t d, bool fp16) {
-  return tokens * hq * d * (32768 + history) > kLongChunk * 32768 && history * (fp16 ? 1 : 16) >= tokens &&
-         (history + 64) * hk * d < (1ll << 31);
-}
 constexpr int64_t kSlotBytes = 64 << 10;  // request table + plan of up to ~1900 items
 constexpr int64_t kAlign = 256;
 
@@ -157,13 +151,11 @@ extern "C" int oscar_decode_step_v1(oscar_context_v1* ctx, oscar_step_args_v1* a
     if ((hist + bs - 1) / bs > a.block_table_cols) return fail(-22, "Block table cannot cover the history");
   }
   if (qsl[0] != 0 || clip(qsl[B]) != n) return OSCAR_STEP_NOT_DECODE;
-  bool prefill = false;
   for (int r = 0; r < B; ++r) {
     const int64_t nq = clip(qsl[r + 1]) - clip(qsl[r]);
     if (nq == 0) continue;
     // chunks of more than 32 rows per KV head run as sub-requests, up to kMaxSplitRows
     if (has_new && nq * G > kMaxSplitRows) return OSCAR_STEP_NOT_DECODE;
-    prefill = prefill || (has_new && prefill_chunk(nq, seqs[r] - nq, hq, hk, d, a.q_dtype == OSCAR_F16));
     if (has_new && seqs[r] == nq) return OSCAR_STEP_NOT_DECODE;  // history-free: prefill
   }
   hipStream_t s = (hipStream_t)stream;
@@ -174,7 +166,6 @@ extern "C" int oscar_decode_step_v1(oscar_context_v1* ctx, oscar_step_args_v1* a
     return fail(-5, "oscar_decode_step_v1: cannot query the stream's capture status");
   if (cap != hipStreamCaptureStatusNone)
     return fail(-22, "oscar_decode_step_v1: eager only (the stream is capturing a graph)");
-  if (prefill) return OSCAR_STEP_NOT_DECODE;  // after the capture check: refused there, as any step
   // ---- ring slot (wait only if the slot's previous call has not finished reading it)
   std::unique_lock<std::mutex> lock(ctx->mu);
   const int slot = ctx->next;

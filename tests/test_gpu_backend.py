@@ -201,56 +201,6 @@ def test_native_step_metadata_follows_every_call(cuda, requests):
     assert excess <= 0
 
 
-@pytest.mark.parametrize("history,tokens,others,qdt,long", [
-    (1100, 990, [], "bf16", False), (1100, 991, [], "bf16", True),       # the line at 6 heads of 256
-    (1100, 991, [700, 129], "bf16", True),                               # beside decodes
-    (1100, 1030, [], "f16", True), (900, 1030, [], "f16", False),        # fp16: a history as long as the chunk
-    (64, 1025, [], "bf16", False), (65, 1025, [], "bf16", True),         # bf16: a sixteenth of it
-], ids=str)
-def test_long_cached_chunks_take_the_prefill(cuda, history, tokens, others, qdt, long):
-    """Both sides of the line between the split-K decode and the prefill for a cached chunk:
-    the native step and the classification agree on the route, and the output is the oracle's."""
-    from oracle.attention import attention_ref
-    from oscar_amd import backend as B
-
-    dev, tdt = torch.device("cuda", 0), torch.bfloat16 if qdt == "bf16" else torch.float16
-    lengths = [tokens] + [1] * len(others)
-    c = cases.make_case([history] + others, lengths, seed=tokens)
-    N, (d, hq, hk) = c["qsl"][-1], (256, 6, 1)
-    batch = B._Batch.classify(c["qsl"], c["seqs"], N, True, hq // hk, hk, d, tdt == torch.float16)
-    assert batch.long == ([0] if long else [])
-    impl, layer = OscarAttentionBackendImplFactory(), _Layer()
-    eye = torch.eye(d, dtype=torch.float32, device=dev)
-    layer._oscar_rots = (eye, eye)
-    caches = [torch.from_numpy(c[x]).view(torch.int8).to(dev) for x in ("k8", "v8")]
-    impl._set_caches(caches)
-    impl._ensure_staging(layer, caches)
-    for arena, x in zip((layer._oscar_stage_k, layer._oscar_stage_v, layer._oscar_slot_owner), c["stage"]):
-        arena.copy_(torch.from_numpy(x))
-    md = _MD()
-    md.num_actual_tokens = N
-    md.slot_mapping = torch.full((N,), -1, dtype=torch.int64, device=dev)
-    md.query_start_loc_cpu = torch.tensor(c["qsl"], dtype=torch.int32)
-    md.seq_lens_cpu = torch.tensor(c["seqs"], dtype=torch.int32)
-    md.block_tables = torch.from_numpy(c["bt"]).to(dev)
-    tq, tk, tv = (torch.from_numpy(c[x]).to(dev).to(tdt).view(N, -1) for x in "qkv")
-    out = torch.full((N, hq * d), float("nan"), dtype=tdt, device=dev)
-    impl.forward(layer, tq, tk, tv, caches, md, output=out)
-    look = B.MANY_TOKENS
-    try:
-        B.MANY_TOKENS = 1 << 30  # no early look: the native step itself declines the batch
-        assert impl._native_step(layer, tq, tk, tv, caches, md, torch.empty_like(out)) == (not long)
-    finally:
-        B.MANY_TOKENS = look
-    ref, _ = attention_ref(c["q"], c["k"], c["v"], c["k8"], c["v8"], c["bt"], c["qsl"], c["seqs"], c["scale"],
-                           c["stage"], q_dtype=qdt)
-    got = out.float().view(N, hq, d).cpu().numpy()
-    # 2e-2 absolute plus one output ulp of the value, as in the tests above
-    excess = float((np.abs(got - ref) - (2e-2 + (2.0 ** -7 if qdt == "bf16" else 2.0 ** -10) * np.abs(ref))).max())
-    print(f"chunk {tokens} over {history}, {qdt}: max|out - oracle| = {np.abs(got - ref).max():.3e}", flush=True)
-    assert excess <= 0
-
-
 def OscarAttentionBackendImplFactory():
     from oscar_amd.backend import OscarAttentionBackendImpl
 
