@@ -28,8 +28,9 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-# the current stream's raw handle without building a Stream object (2 us a call)
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# the current stream's raw handle without building a Stream object (2 us a call); a torch
+# built without a GPU has none, and imports this module all the same
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(device: torch.device) -> int:
