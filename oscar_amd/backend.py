@@ -37,10 +37,12 @@ from .rotation import get_layer_rotation
 
 MAX_DECODE_ROWS = 32  # rows (query tokens x heads per KV head) of one decode MFMA tile
 # A cached chunk of more rows per KV head runs through the split-K decode as
-# sub-requests of MAX_DECODE_ROWS rows (each streams the request's history once), up to
-# this many rows; longer chunks go to the MFMA prefill, which decodes the history once
-# and shares it between query tiles but walks it serially per query tile (at 24576
-# history tokens: 24-156 us for chunks of 8-400 tokens against 1.1 ms).
+# sub-requests of MAX_DECODE_ROWS rows (each decodes the request's history once), up to
+# this many rows; longer chunks go to the MFMA prefill, which decodes the history once for
+# all.  The prefill is the faster one well below the line (6 heads of 256, split-K / prefill
+# in us: 400 tokens over 15000 132 / 141, 800 284 / 178, 2700 772 / 391), but its history V
+# values are rounded to bf16 and the split-K decode's are not: single outputs move by up to
+# 0.34 of the outputs' root mean square where a chunk changes route.
 MAX_SPLIT_ROWS = 32 * 512
 # Calls of more new tokens than this are looked over for prompts before the native step's
 # arguments are built (about 30 us that a batch with a prompt throws away; decode and

@@ -307,7 +307,7 @@ __device__ __forceinline__ void hold_acc(f32x16 (&o)[N]) {
 // per 256 rows x 32 keys (2048 of MFMA) at the 1.9 GHz the power allows.  The call with
 // its other launches: 1900 us before (four waves of 32 rows, tiles through registers, one
 // phase after the other), 1230 us now, 0.92 PFLOP/s; a large library bf16 product reaches
-// 1.2 on this card.
+// 1.2 to 1.36 on this card.
 template <int D, int QT, int NB>
 __global__ __launch_bounds__(kThreads, prefill_wgs(D, NB)) void prefill_kernel(PrefillParams P) {
   using QV = typename QVec<QT>::type;    // one MFMA operand in the query dtype
