@@ -323,3 +323,20 @@ def test_prompts_are_found_before_the_native_step(seed):
         else:
             batch = B._Batch.classify(qsl, seqs, actual, True, group)
             assert got == bool(batch.fresh or batch.long)
+
+
+@pytest.mark.parametrize("hq,hk,d,tokens,length", [(6, 1, 256, 2048, 32768), (16, 2, 128, 4096, 8192),
+                                                   (24, 4, 256, 512, 4096), (6, 1, 256, 15360, 24616)])
+def test_prefill_reserve_bounds_every_shorter_call(hq, hk, d, tokens, length):
+    """The reserved prefill workspace covers every call of up to that many tokens over a
+    history that fits (a shorter call can split further than the longest)."""
+    import random
+    from oscar_amd import _lib, integration
+
+    bytes_of = _lib.load().oscar_prefill_workspace_bytes_v2
+    impl = NS(num_heads=hq, num_kv_heads=hk, head_size=d)
+    reserve = integration.transient_parts(impl, tokens, length)["prefill"]
+    r = random.Random(hq * d)
+    for _ in range(3000):
+        n = r.randint(1, tokens)
+        assert bytes_of(r.choice([0, r.randint(0, length - n)]), n, hq, hk, d) <= reserve
