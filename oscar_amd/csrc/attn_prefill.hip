@@ -351,7 +351,7 @@ __global__ __launch_bounds__(kThreads, prefill_wgs(D, NB)) void prefill_kernel(P
   const int64_t q0 = (int64_t)qt * P.qtok;
   const int64_t q1 = (q0 + P.qtok < A.num_tokens) ? q0 + P.qtok : A.num_tokens;
   // this wave's own key tiles end at ke_own: the lighter tile of a pair may see fewer, and
-  // must not multiply values past them (0 x inf)
+  // must not multiply values past them (0 x inf; in the last of them see pv)
   int ke_own = (int)tile_keys(hist, q1);
   ke_own = !live || ke_own <= kb ? kb + 1 : ke_own < ke ? ke_own : ke;
 
@@ -622,15 +622,25 @@ __global__ __launch_bounds__(kThreads, prefill_wgs(D, NB)) void prefill_kernel(P
   };
   // ---- O^T += V^T P^T of the tile before, whose first V operands are in va, beside the
   // probabilities and row sums of this tile (SM); reads the first K operands of the tile
-  // at `koff`
+  // at `koff`.  Without SM: the wave's last tile, in which values of keys past its query
+  // tile (a later tile's, and the pair's other tile reads them) are taken as zero: their
+  // probabilities are, but an infinite value's product would be NaN.
   auto pv = [&](unsigned off, unsigned koff, auto sm) __attribute__((always_inline)) {
     constexpr bool SM = decltype(sm)::value;
     constexpr int NPV = D / 16;   // steps
     constexpr int EPS = 16 / NPV; // elements of S per row block and step
     float nm[NB], pe[NB][2];
+    u32x4 seen[2] = {};  // all ones where the step's V operand is of a key of this wave's tile
     if constexpr (SM) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) { nm[nb] = neg_m(nb); lsum[nb] = 0.f; }
+    } else {
+      const int lim = (int)(hist + q1) - (ke_own - 1) * kKeys - 4 * (int)(fresh(ulane) >> 5);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {  // keys 16 s + 8 h + 4 g + (e & 3)
+        const int key = 16 * (e >> 3) + 8 * (e >> 2 & 1) + (e & 3);
+        seen[e >> 3][e / 2 % 4] |= key < lim ? 0xffffu << 16 * (e & 1) : 0u;
+      }
     }
     auto pair_done = [&](int nb, int r) __attribute__((always_inline)) {  // elements r - 1, r
       lsum[nb] += pe[nb][0] + pe[nb][1];
@@ -640,7 +650,9 @@ __global__ __launch_bounds__(kThreads, prefill_wgs(D, NB)) void prefill_kernel(P
     for (int i = 0; i < NPV; ++i) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
-        O[nb][i >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[i % VA], __builtin_bit_cast(f16x8, p_cur[nb][i & 1]), O[nb][i >> 1], 0, 0, 0);
+        f16x8 v = va[i % VA];
+        if constexpr (!SM) v = __builtin_bit_cast(f16x8, __builtin_bit_cast(u32x4, v) & seen[i & 1]);
+        O[nb][i >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, __builtin_bit_cast(f16x8, p_cur[nb][i & 1]), O[nb][i >> 1], 0, 0, 0);
         if (nb == 0 && i + VA - 1 < NPV) va[(i + VA - 1) % VA] = v_op(off, i + VA - 1);
         if (SM && nb == NB - 1 && i == NPV - 1) k_ahead(koff);
         if constexpr (SM) {

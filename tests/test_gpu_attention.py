@@ -378,19 +378,37 @@ def test_prefill_tile_edges_match_oracle(cuda, prefix, n, d, hk, group, qdt, spl
     assert excess <= 0 and d_lse <= 1e-3
 
 
-def test_prefill_values_past_a_tile_do_not_reach_it(cuda):
-    """inf in the values of the last tokens: the rows of earlier query tiles, which do not
-    see them, stay as they are, also in the tile that shares a workgroup with the last."""
+@pytest.mark.parametrize("prefix,n,d,hk,group,first,bad,qdt", [
+    (0, 2600, 256, 1, 32, 2592, np.inf, "bf16"),   # paired query tiles of 4 tokens; a key tile of its own
+    (0, 2600, 256, 1, 32, 2596, np.inf, "bf16"),   # the last query tile only: its pair mate shares the key tile
+    (0, 2600, 256, 1, 32, 2597, np.nan, "f16"),
+    (0, 5003, 256, 1, 6, 4790, 2.0 ** 24, "bf16"), # finite, past the range of the PV form
+    (0, 100, 256, 1, 6, 25, np.inf, "bf16"),       # one tile of 21 tokens per workgroup, key tile 0 shared
+    (0, 60, 128, 2, 8, 17, np.inf, "f16"),
+    (45, 100, 256, 1, 6, 21, np.nan, "bf16"),      # a key tile of history and chunk rows
+    (1037, 900, 256, 1, 6, 700, np.inf, "bf16")])  # the last of a query tile's chunks
+def test_prefill_values_past_a_tile_do_not_reach_it(cuda, prefix, n, d, hk, group, first, bad, qdt):
+    """Values that overflow (or NaN) from token `first` on: the rows of the query tiles
+    before its own, which do not see them, keep every bit, also where a key tile or a
+    workgroup is shared with a later query tile."""
     from oscar_amd import ops
 
-    n, group = 2600, 32  # 650 query tiles of 4 tokens: paired
-    q, k, v = (cases.bf16_normal((n, h, 256), 90 + h) for h in (group, 1, 1))
-    clean = ops.attention_prefill(dev(q), dev(k), dev(v), 1 / 16, head_dim=256)
-    v[2592:] = np.inf  # the last two query tiles, in one key tile of their own
-    got = ops.attention_prefill(dev(q), dev(k), dev(v), 1 / 16, head_dim=256)
+    c = cases.make_case([prefix], [n], fresh=True, seed=n + first, hk=hk, group=group, d=d)
+    tdt = torch.float16 if qdt == "f16" else torch.bfloat16
+    kw = dict(head_dim=d)
+    if prefix:
+        kw.update(history=prefix, k_cache=torch.from_numpy(c["k8"]).view(torch.int8).cuda(),
+                  v_cache=torch.from_numpy(c["v8"]).view(torch.int8).cuda(),
+                  block_table_row=torch.from_numpy(c["bt"][0]).cuda())
+    q, k, v = (dev(c[x], tdt) for x in "qkv")
+    clean = ops.attention_prefill(q, k, v, c["scale"], **kw)
+    v[first:] = bad
+    got = ops.attention_prefill(q, k, v, c["scale"], **kw)
     torch.cuda.synchronize()
-    assert torch.equal(got[:2592], clean[:2592])
-    assert not torch.isfinite(got[2596:].float()).any()
+    qtok = 128 // group
+    before, after = first // qtok * qtok, -(-first // qtok) * qtok
+    assert before > 0 and torch.equal(got[:before], clean[:before])
+    assert not torch.isfinite(got[after:].float()).any()
 
 
 def test_prefill_fp16_queries(cuda):
