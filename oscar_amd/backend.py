@@ -407,16 +407,18 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
         """The batch holds a history-free request or a chunk past MAX_SPLIT_ROWS, which the
         native step leaves to the general path.  False as well for a batch that the native
         step refuses: its checks come first, and it words the errors."""
-        table = _block_tables(md)
         group, bs = self.num_heads // self.num_kv_heads, self.key_cache.shape[1]
-        if group > MAX_DECODE_ROWS or table.ndim != 2 or table.shape[0] < len(qsl) - 1 or table.shape[1] < 1:
+        starts = np.minimum(np.asarray(qsl), n, dtype=np.int64)
+        chunks = starts[1:] - starts[:-1]
+        lens = np.asarray(seqs)[:len(chunks)]
+        if not ((chunks == lens) & (chunks > 0)).any() \
+                and (n * group <= MAX_SPLIT_ROWS or int(chunks.max()) * group <= MAX_SPLIT_ROWS):
+            return False  # every decode and verify step (a walk over 512 requests took 80 us)
+        table = _block_tables(md)
+        if group > MAX_DECODE_ROWS or table.ndim != 2 or table.shape[0] < len(chunks) or table.shape[1] < 1:
             return False
-        starts, found = [min(s, n) for s in qsl.tolist()], False
-        for a, b, seq in zip(starts, starts[1:], seqs.tolist()):
-            if b < a or seq < 0 or b > a and (seq < b - a or -(-(seq - (b - a)) // bs) > table.shape[1]):
-                return False
-            found = found or b > a and (seq == b - a or (b - a) * group > MAX_SPLIT_ROWS)
-        return found
+        uncovered = (lens < chunks) | (-(-(lens - chunks) // bs) > table.shape[1])
+        return not ((chunks < 0).any() or (lens < 0).any() or (uncovered & (chunks > 0)).any())
 
     def _step_args(self, layer, device, dtype, scratch):
         """The layer's step arguments that stay fixed from call to call (caches, window

@@ -340,3 +340,27 @@ def test_prefill_reserve_bounds_every_shorter_call(hq, hk, d, tokens, length):
     for _ in range(3000):
         n = r.randint(1, tokens)
         assert bytes_of(r.choice([0, r.randint(0, length - n)]), n, hq, hk, d) <= reserve
+
+
+@pytest.mark.parametrize("requests,tokens", [(129, 1), (512, 1), (64, 4), (300, 2)])
+def test_decode_steps_are_not_walked_for_prompts(requests, tokens):
+    """A decode or verify step of many tokens holds no prompt: found without a Python list
+    of its requests or a look at its block tables."""
+    import numpy as np
+    from oscar_amd import backend as B
+
+    class Array(np.ndarray):
+        def tolist(self):
+            raise AssertionError("walked")
+
+        __iter__ = tolist
+
+    impl = B.OscarAttentionBackendImpl.__new__(B.OscarAttentionBackendImpl)
+    impl.num_heads, impl.num_kv_heads, impl.key_cache = 6, 1, torch.empty(4, 128, 1, 1)
+    qsl = np.arange(0, tokens * requests + 1, tokens, dtype=np.int32).view(Array)
+    seqs = np.full(requests + 3, 300, np.int32).view(Array)
+    seqs[-3:] = 0  # padding
+    assert not impl._has_prompt(NS(), qsl, seqs, tokens * requests)
+    seqs = np.asarray(seqs)
+    seqs[requests - 1] = tokens  # one of them has no history after all
+    assert impl._has_prompt(NS(block_tables=torch.zeros(requests, 8)), np.asarray(qsl), seqs, tokens * requests)
