@@ -854,13 +854,18 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams P) {
     A.lse[qi * A.num_q_heads + head] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
 }
 
-// Two query tiles per workgroup from this many units on.  Below it the chip is not full
-// with one tile each (2048 fresh tokens are 247 units), and a unit's latency counts: one
-// tile takes about two thirds of a pair's time per key tile.  Above it pairs halve the
-// operand reads per MFMA (15360 + 9256 tokens: 1.23 ms against 1.60 ms unpaired).  At head
-// dim 128 two unpaired workgroups fit a CU and overlap each other (8000 + 4000 tokens, 16
-// heads on 2: 374 us against 380 us paired), so there are no pairs there.
-constexpr int64_t kPairUnits = 512;
+// Two query tiles per workgroup from this many units on (head dim 256, where a CU holds one
+// workgroup).  One tile takes about two thirds of a pair's time per key tile, so up to one
+// unit per CU a unit's latency counts; beyond it the unpaired units need a second round of
+// the chip, which pairs do without up to 512 and halve the operand reads per MFMA after.
+// The line lies an eighth above a round, since the last units in launch order are the short
+// ones.  Unpaired / paired in us: fresh tokens of 6 heads on 1, 2048 (247 units) 44 / 53,
+// 2200 (283) 53 / 55, 2400 (333) 67 / 55, 3000 (473) 76 / 63, 6000 (625) 196 / 178; 12 heads
+// on 2, 1500 (288) 53 / 53, 1800 (398) 68 / 57; 8000 + 1600 (500) 144 / 121; 15360 + 9256
+// 1.60 / 1.23 ms.  At head dim 128 two unpaired workgroups fit a CU and overlap each other
+// (8000 + 4000 tokens, 16 heads on 2: 374 us against 380 us paired), so there are no pairs
+// there.
+constexpr int64_t kPairUnits = kSplitCUs + kSplitCUs / 8;
 template <int D, int QT>
 void launch_prefill(const PrefillParams& p, dim3 grid, bool pairs, hipStream_t s) {
   if constexpr (D == 256) {

@@ -341,6 +341,8 @@ def test_prefill_split_matches_unsplit_and_oracle(cuda, prefix, n, d, hk, group,
     (1037, 5003, 256, 1, 16, "bf16"), # paired, a key tile of history and chunk rows
     (1037, 5003, 256, 1, 16, "f16"),
     (513, 3001, 256, 7, 3, "bf16"),   # paired, the lighter tile ends key tiles before the other
+    (0, 2226, 256, 1, 6, "bf16"),     # the last size of one tile per workgroup and the first of two
+    (0, 2227, 256, 1, 6, "bf16"),
     (0, 257, 256, 3, 1, "bf16"),      # one tile per workgroup, 128 tokens a tile
     (95, 33, 256, 1, 6, "bf16"),      # one or two key tiles of everything
     (1037, 3003, 128, 2, 8, "bf16"), (0, 4001, 128, 2, 8, "f16"), (40, 1, 128, 1, 5, "f16")])
