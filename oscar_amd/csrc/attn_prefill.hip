@@ -240,12 +240,12 @@ __global__ __launch_bounds__(256) void history_bf16_kernel(PrefillParams P) {
 // The wait is the caller's (vmcnt): the builtin form would make the compiler drain every
 // load before each later LDS read.
 __device__ __forceinline__ void dma16(unsigned lds, const void* addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(addr) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(addr) : "m0", "memory");
 }
 
 // the same with a uniform base and a 32-bit byte offset
 __device__ __forceinline__ void dma16(unsigned lds, uint64_t base, unsigned voff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "m0", "memory");
 }
 
 // Every wave's LDS traffic is done and all but the last PENDING of this wave's DMA

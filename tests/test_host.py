@@ -364,3 +364,15 @@ def test_decode_steps_are_not_walked_for_prompts(requests, tokens):
     seqs = np.asarray(seqs)
     seqs[requests - 1] = tokens  # one of them has no history after all
     assert impl._has_prompt(NS(block_tables=torch.zeros(requests, 8)), np.asarray(qsl), seqs, tokens * requests)
+
+
+def test_asm_that_writes_m0_says_so():
+    """Inline assembly that sets m0 lists it as clobbered: the compiler may keep a value of
+    its own there."""
+    import re
+    from pathlib import Path
+    import oscar_amd
+
+    statements = [s for f in sorted((Path(oscar_amd.__file__).parent / "csrc").iterdir())
+                  for s in re.findall(r"\basm\b[^;]*;", f.read_text()) if re.search(r"s_mov_b32 m0\b", s)]
+    assert statements and all('"m0"' in s for s in statements)
