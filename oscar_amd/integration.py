@@ -148,11 +148,10 @@ def transient_parts(impl, max_tokens: int, max_model_len: int = 0, max_seqs: int
     lib = _lib_sizes()
     hq, hk, d = impl.num_heads, impl.num_kv_heads, impl.head_size
     items = decode_items_bound(max_tokens, max_model_len, hk, hq // hk, max_seqs)
-    prefill = max(0, lib.oscar_prefill_workspace_bytes_v2(max(max_model_len, 0), max_tokens, hq, hk, d))
-    if prefill > 0:
-        tiles = -(-max_tokens // (128 // (hq // hk)))
-        history = lib.oscar_prefill_workspace_bytes_v1(max(max_model_len, 0), hk, d)
-        prefill = max(prefill, history + 256 + (512 + tiles * hk) * 128 * (d + 1) * 4)
+    prefill, length = 0, max(max_model_len, 0)
+    if lib.oscar_prefill_workspace_bytes_v2(length, max_tokens, hq, hk, d) >= 0:  # a shape the prefill takes
+        slots = 512 + -(-max_tokens // (128 // (hq // hk))) * hk
+        prefill = lib.oscar_prefill_workspace_bytes_v1(length, hk, d) + 256 + slots * 128 * (d + 1) * 4
     return {
         "store": lib.oscar_store_workspace_bytes_v1(max_tokens, hk, d),
         "step": lib.oscar_step_workspace_bytes_v1(max_tokens, hq, hk, d, items),

@@ -326,10 +326,12 @@ def test_prompts_are_found_before_the_native_step(seed):
 
 
 @pytest.mark.parametrize("hq,hk,d,tokens,length", [(6, 1, 256, 2048, 32768), (16, 2, 128, 4096, 8192),
-                                                   (24, 4, 256, 512, 4096), (6, 1, 256, 15360, 24616)])
+                                                   (24, 4, 256, 512, 4096), (6, 1, 256, 15360, 24616),
+                                                   (6, 1, 256, 32768, 0), (24, 4, 256, 15360, 0)])
 def test_prefill_reserve_bounds_every_shorter_call(hq, hk, d, tokens, length):
     """The reserved prefill workspace covers every call of up to that many tokens over a
-    history that fits (a shorter call can split further than the longest)."""
+    history that fits (a shorter call can split further than the longest, which may not
+    split at all; length 0: the model's length is not known)."""
     import random
     from oscar_amd import _lib, integration
 
@@ -339,7 +341,7 @@ def test_prefill_reserve_bounds_every_shorter_call(hq, hk, d, tokens, length):
     r = random.Random(hq * d)
     for _ in range(3000):
         n = r.randint(1, tokens)
-        assert bytes_of(r.choice([0, r.randint(0, length - n)]), n, hq, hk, d) <= reserve
+        assert bytes_of(r.choice([0, r.randint(0, max(length - n, 0))]), n, hq, hk, d) <= reserve
 
 
 @pytest.mark.parametrize("requests,tokens", [(129, 1), (512, 1), (64, 4), (300, 2)])
