@@ -144,13 +144,16 @@ def transient_parts(impl, max_tokens: int, max_model_len: int = 0, max_seqs: int
     item partials), the general decode's item partials, and the continuation prefill's
     (the bf16 history of up to max_model_len tokens and the partials of its split over
     up to max_tokens query tokens: shorter calls can split further than the longest one, into
-    at most 512 chunks of work and one more per query tile of 128 rows)."""
+    at most 512 chunks of work and one more per query tile of 128 rows, and no tile into more
+    than 32 or into chunks of fewer than 512 keys)."""
     lib = _lib_sizes()
     hq, hk, d = impl.num_heads, impl.num_kv_heads, impl.head_size
     items = decode_items_bound(max_tokens, max_model_len, hk, hq // hk, max_seqs)
     prefill, length = 0, max(max_model_len, 0)
     if lib.oscar_prefill_workspace_bytes_v2(length, max_tokens, hq, hk, d) >= 0:  # a shape the prefill takes
-        slots = 512 + -(-max_tokens // (128 // (hq // hk))) * hk
+        tiles = -(-max_tokens // (128 // (hq // hk))) * hk
+        chunks = min(32, -(-(length + max_tokens) // 512))  # of a tile
+        slots = min(512 + tiles, tiles * chunks) if chunks > 1 else 0
         prefill = lib.oscar_prefill_workspace_bytes_v1(length, hk, d) + 256 + slots * 128 * (d + 1) * 4
     return {
         "store": lib.oscar_store_workspace_bytes_v1(max_tokens, hk, d),

@@ -344,6 +344,19 @@ def test_prefill_reserve_bounds_every_shorter_call(hq, hk, d, tokens, length):
         assert bytes_of(r.choice([0, r.randint(0, max(length - n, 0))]), n, hq, hk, d) <= reserve
 
 
+@pytest.mark.parametrize("hq,hk,d,tokens,length", [(6, 1, 256, 64, 32768), (16, 2, 128, 16, 4096), (24, 4, 256, 300, 400),
+                                                   (32, 1, 256, 64, 9000)])
+def test_prefill_reserve_of_a_small_budget_is_small(hq, hk, d, tokens, length):
+    """A small token budget reserves no more than twice what its calls can use (and the
+    256-byte rounding): a query tile has at most 32 chunks, of at least 16 key tiles."""
+    from oscar_amd import _lib, integration
+
+    bytes_of = _lib.load().oscar_prefill_workspace_bytes_v2
+    reserve = integration.transient_parts(NS(num_heads=hq, num_kv_heads=hk, head_size=d), tokens, length)["prefill"]
+    used = max(bytes_of(h, n, hq, hk, d) for n in range(1, tokens + 1) for h in {0, length // 2, length - n, length})
+    assert used <= reserve <= 2 * used + 256
+
+
 @pytest.mark.parametrize("requests,tokens", [(129, 1), (512, 1), (64, 4), (300, 2)])
 def test_decode_steps_are_not_walked_for_prompts(requests, tokens):
     """A decode or verify step of many tokens holds no prompt: found without a Python list
