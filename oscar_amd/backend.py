@@ -533,7 +533,8 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
                                   outputs=cached, **extra)
 
         # ---- read
-        if actual < q3.shape[0] or actual == 0 or not batch.writes_all(has_new):
+        if actual < q3.shape[0] or actual == 0 or not batch.writes_all(has_new) \
+                or not batch.decode_only and actual * hq * d < output.numel():
             output.zero_()
         if actual == 0:
             return output

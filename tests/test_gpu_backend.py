@@ -201,6 +201,59 @@ def test_native_step_metadata_follows_every_call(cuda, requests):
     assert excess <= 0
 
 
+# name: histories, chunks, and rows that belong to no request: before the first one, after
+# the last one, past num_actual_tokens, and of the output alone
+ROW_LAYOUTS = {
+    "prompts": ([0, 0], [300, 41], 0, 0, 0, 0),
+    "prompts, output of more rows": ([0, 0], [300, 41], 0, 0, 0, 9),
+    "mixed, empty requests": ([700, 0, 300, 0, 129, 0], [3, 0, 0, 250, 1, 40], 0, 0, 0, 0),
+    "mixed, output of more rows": ([700, 0], [3, 150], 0, 0, 0, 2),
+    "mixed, padded query": ([700, 0], [3, 150], 0, 0, 7, 0),
+    "mixed, rows before and after": ([0, 700], [150, 30], 3, 5, 0, 0),
+    "prompt, rows after": ([0], [200], 0, 56, 0, 0),
+}
+
+
+@pytest.mark.parametrize("name", ROW_LAYOUTS)
+def test_output_rows_are_written_or_zero(cuda, name):
+    """The general path on an output full of NaN: a request's rows hold what the batch
+    without any other rows gives, and every other row is zero."""
+    prefixes, lengths, front, tail, pad, extra = ROW_LAYOUTS[name]
+    dev = torch.device("cuda", 0)
+    d, hq, hk = 256, 6, 1
+    c = cases.make_case(prefixes, lengths, fresh=True, seed=41)
+    used = c["qsl"][-1]
+    eye = torch.eye(d, dtype=torch.float32, device=dev)
+
+    def run(front, tail, pad, extra, fill):
+        impl, layer = OscarAttentionBackendImplFactory(), _Layer()
+        layer._oscar_rots = (eye, eye)
+        caches = [torch.from_numpy(c[x]).view(torch.int8).to(dev).clone() for x in ("k8", "v8")]
+        impl._set_caches(caches)
+        impl._ensure_staging(layer, caches)
+        for arena, x in zip((layer._oscar_stage_k, layer._oscar_stage_v, layer._oscar_slot_owner), c["stage"]):
+            arena.copy_(torch.from_numpy(x))
+        actual = front + used + tail
+        md = _MD()
+        md.num_actual_tokens = actual
+        md.slot_mapping = torch.full((actual,), -1, dtype=torch.int64, device=dev)
+        md.query_start_loc_cpu = torch.tensor([front + x for x in c["qsl"]], dtype=torch.int32)
+        md.seq_lens_list = list(c["seqs"])
+        md.block_tables = torch.from_numpy(c["bt"]).to(dev)
+        rows = [torch.ones(actual + pad, h * d, dtype=torch.bfloat16, device=dev) for h in (hq, hk, hk)]
+        for x, name in zip(rows, "qkv"):
+            x[front:front + used] = torch.from_numpy(c[name]).to(dev).bfloat16().view(used, -1)
+        out = torch.full((actual + pad + extra, hq * d), fill, dtype=torch.bfloat16, device=dev)
+        impl._run(layer, *rows, caches, md, out, write=True)
+        torch.cuda.synchronize()
+        return out
+
+    want = run(0, 0, 0, 0, 0.0)
+    got = run(front, tail, pad, extra, float("nan"))
+    assert torch.equal(got[front:front + used], want)
+    assert (got[:front] == 0).all() and (got[front + used:] == 0).all()
+
+
 def OscarAttentionBackendImplFactory():
     from oscar_amd.backend import OscarAttentionBackendImpl
 

@@ -283,6 +283,24 @@ def test_mixed_batch_routes_slice_consecutive_decodes_and_gather_otherwise():
     assert impl._decode_route(b3)["qsl"] == [0, 4, 4, 5]
 
 
+@pytest.mark.parametrize("qsl,seqs,actual,has_new,group,whole", [
+    ([0, 300, 341], [300, 41], 341, True, 6, True),              # prompts
+    ([0, 3, 3, 253, 254], [703, 300, 250, 130], 254, True, 6, True),  # an empty request between
+    ([3, 153, 183], [150, 730], 183, True, 6, False),            # rows before the first request
+    ([0, 150, 180], [150, 730], 185, True, 6, False),            # rows after the last
+    ([0, 200, 256], [200, 0], 200, True, 6, True),               # padded starts past the tokens
+    ([0, 4, 2, 8], [104, 0, 206], 8, True, 6, False),            # starts that fall back
+    ([0, 20000], [30000], 20000, True, 6, True),                 # a long chunk
+    ([0, 4], [104], 4, True, 40, True),                          # heads past a decode tile: long
+    ([0, 4], [104], 4, False, 40, False),                        # without new tokens nobody writes it
+    ([0, 4], [104], 4, False, 6, True)])
+def test_writes_all_knows_the_rows_of_no_request(qsl, seqs, actual, has_new, group, whole):
+    """The output is cleared unless the requests' rows tile it and each of them is written."""
+    from oscar_amd.backend import _Batch
+
+    assert _Batch.classify(qsl, seqs, actual, has_new, group).writes_all(has_new) == whole
+
+
 @pytest.mark.parametrize("seed", range(6))
 def test_prompts_are_found_before_the_native_step(seed):
     """The early look for prompts sends a batch down the general path exactly where the
