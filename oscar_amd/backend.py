@@ -553,7 +553,9 @@ class OscarAttentionBackendImpl(BaseAttentionImpl):  # type: ignore[misc,valid-t
             v_rot = None if v3 is None else ops.rotate(v3[:actual], rv)
         stage = self._stage(layer)
         table = _block_tables(md)
-        out_rot = torch.empty(actual, hq, d, dtype=torch.float32, device=dev)
+        # rows that nothing writes are rotated with the others: zeros stay zeros
+        new_rows = torch.empty if batch.writes_all(has_new) else torch.zeros
+        out_rot = new_rows(actual, hq, d, dtype=torch.float32, device=dev)
         lse = torch.empty(actual, hq, dtype=torch.float32, device=dev)
         if plan is not None:
             if route["identity"]:

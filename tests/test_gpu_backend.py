@@ -211,6 +211,8 @@ ROW_LAYOUTS = {
     "mixed, padded query": ([700, 0], [3, 150], 0, 0, 7, 0),
     "mixed, rows before and after": ([0, 700], [150, 30], 3, 5, 0, 0),
     "prompt, rows after": ([0], [200], 0, 56, 0, 0),
+    "decodes, rows after": ([700, 300], [1, 40], 0, 3, 2, 0),
+    "decodes, rows before": ([700, 300], [1, 40], 2, 0, 0, 0),
 }
 
 
@@ -252,6 +254,36 @@ def test_output_rows_are_written_or_zero(cuda, name):
     got = run(front, tail, pad, extra, float("nan"))
     assert torch.equal(got[front:front + used], want)
     assert (got[:front] == 0).all() and (got[front + used:] == 0).all()
+
+
+def test_unread_long_requests_leave_zeros(cuda, monkeypatch):
+    """More heads per KV head than a decode tile takes, without new tokens: nothing reads
+    such a request, so its rows are zero (not the rotation of memory that nothing wrote)."""
+    dev = torch.device("cuda", 0)
+    d, hq = 256, 40
+    c = cases.make_case([300, 500], [4, 60], group=hq, fresh=False, seed=43)
+    impl, layer = OscarAttentionBackendImplFactory(), _Layer()
+    impl.num_heads = hq
+    eye = torch.eye(d, dtype=torch.float32, device=dev)
+    layer._oscar_rots = (eye, eye)
+    caches = [torch.from_numpy(c[x]).view(torch.int8).to(dev) for x in ("k8", "v8")]
+    impl._set_caches(caches)
+    md = _MD()
+    md.num_actual_tokens = 64
+    md.query_start_loc_cpu = torch.tensor(c["qsl"], dtype=torch.int32)
+    md.seq_lens_list = list(c["seqs"])
+    md.block_tables = torch.from_numpy(c["bt"]).to(dev)
+    out = torch.full((64, hq * d), float("nan"), dtype=torch.bfloat16, device=dev)
+    empty = torch.empty
+
+    def holding_nan(*shape, **kw):
+        x = empty(*shape, **kw)
+        return x.fill_(float("nan")) if x.is_floating_point() else x
+
+    monkeypatch.setattr(torch, "empty", holding_nan)
+    impl._streaming_attention(layer, torch.from_numpy(c["q"]).to(dev).bfloat16().view(64, -1), None, None, caches, md, out)
+    torch.cuda.synchronize()
+    assert (out == 0).all()
 
 
 def OscarAttentionBackendImplFactory():
