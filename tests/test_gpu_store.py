@@ -368,6 +368,38 @@ def test_store_window_odd_geometry(cuda, qsl, seqs, clips):
     assert_read_copy(v_rot.float().cpu().numpy(), v, rv, n)
 
 
+@pytest.mark.parametrize("clips", [(0.0, 0.0), (0.96, 0.92)])
+@pytest.mark.parametrize("n", [23, 64, 65, 300, 1500])
+@pytest.mark.parametrize("d,hk,dtype", [(256, 1, torch.bfloat16), (128, 2, torch.float16)])
+def test_store_window_does_not_need_the_read_copies(cuda, d, hk, dtype, n, clips):
+    """The window write of fresh prompts asks for no rotated copies: bytes, tags and FP32
+    window are those of the call that does, bit for bit."""
+    from oscar_amd import ops
+    from oscar_amd._lib import STAGE_WRITE
+
+    bs, nb = 128, 24
+    k, v, q = (to_dev(cases.kv_outliers(n, h, d, 57 + h), dtype) for h in (hk, hk, 6 * hk))
+    rk, rv = (torch.from_numpy(cases.qr_rotation(d, x)).cuda() for x in (58, 59))
+    slots = torch.from_numpy(slot_mapping(n, nb * bs, 60)).cuda()
+    st = Staging(bs, hk, d, 128, 256, 8192)
+    st.owner[:] = np.arange(st.rows)[:, None]
+    results = []
+    for copies in (True, False):
+        caches = [cache_dev(x) for x in cases.empty_caches(nb, bs, hk, d)]
+        stage = tuple(torch.from_numpy(a.copy()).cuda() for a in st.arrays())
+        extra = {}
+        if copies:
+            extra = dict(query=q, query_rot=torch.empty_like(q), key_rot=torch.empty_like(k), value_rot=torch.empty_like(v))
+        ops.store(k, v, *caches, slots, head_dim=d, rk=rk, rv=rv, stage=stage, stage_mode=STAGE_WRITE,
+                  qsl_dev=torch.tensor([0, n // 3, n], dtype=torch.int32, device="cuda"),
+                  seqs_dev=torch.tensor([n // 3, n - n // 3], dtype=torch.int32, device="cuda"), num_reqs=2,
+                  recent_tokens=256, sink_tokens_eff=128, k_clip=clips[0], v_clip=clips[1], **extra)
+        torch.cuda.synchronize()
+        results.append((*caches, *stage))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    assert (results[0][0] != 0).any()
+
+
 @pytest.mark.parametrize("n", [23, 1500])  # one-launch path / three launches
 def test_store_capacity_past_31_bits(cuda, n):
     """A cache of 2^31 + 2048 slots, where the kernels split slots into block and offset
