@@ -301,14 +301,16 @@ def test_writes_all_knows_the_rows_of_no_request(qsl, seqs, actual, has_new, gro
     assert _Batch.classify(qsl, seqs, actual, has_new, group).writes_all(has_new) == whole
 
 
+@pytest.mark.parametrize("walked", [True, False])
 @pytest.mark.parametrize("seed", range(6))
-def test_prompts_are_found_before_the_native_step(seed):
+def test_prompts_are_found_before_the_native_step(seed, walked, monkeypatch):
     """The early look for prompts sends a batch down the general path exactly where the
     native step would hand it back (a fresh request or a chunk past MAX_SPLIT_ROWS) and
     leaves every batch that the native step refuses to it."""
     import numpy as np
     from oscar_amd import backend as B
 
+    monkeypatch.setattr(B, "MANY_REQUESTS", 24 if walked else 0)
     r = np.random.default_rng(seed)
     impl = B.OscarAttentionBackendImpl.__new__(B.OscarAttentionBackendImpl)
     impl.num_kv_heads, impl.key_cache = 1, torch.empty(4, 128, 1, 1)
