@@ -29,8 +29,8 @@ constexpr int kRows = 128;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kLazy = 10;     // log2 of the largest row sum of a tile's probabilities before O is rescaled
-// workgroups per CU the register budget of prefill_kernel<D, ., NB> is set for
-constexpr int prefill_wgs(int D, int NB) { return D == 256 ? 1 : 2; }
+// workgroups per CU the register budget of prefill_kernel<D> is set for
+constexpr int prefill_wgs(int D) { return D == 256 ? 1 : 2; }
 // PV runs on v_mfma_f32_32x32x16_f16 with P and V in fp16 for both query dtypes.  bf16
 // V values (8-bit significands) are held as fp16(v * 2^-kVShift): exact for |v| from
 // 2^-6 up to 2^23 (below, within 2^-17 absolutely), and O is scaled back by 2^kVShift.
@@ -141,8 +141,11 @@ SplitPlan plan_split(int64_t hist, int64_t n, int64_t qtok, int64_t hk) {
   const int64_t kmax = kt(ntq - 1);
   int64_t U = (work * hk + kSplitCUs * kUnitsPerCU - 1) / (kSplitCUs * kUnitsPerCU);
   // a little over half a CU's share: the longest units, dispatched first, then fit one round
-  // of the chip with the shorter ones filling the rest.  15360 + 9256 tokens: 1231 us;
-  // exactly the share 1287 us, two thirds of it 1391 us, half of it 1300 us.
+  // of the chip with the shorter ones filling the rest.  Exactly the share / with the term, in
+  // us: 15360 + 9256 tokens of 6 heads on 1 1124 / 1050, 1600 over 8000 148 / 119, 3500 fresh
+  // 102 / 72, 6000 fresh 169 / 175, 12 heads on 2, 3000 fresh 122 / 113, 24 on 4, 1600 fresh
+  // 84 / 87, 8 heads of 128 on 1, 4000 fresh 76 / 64, 16 on 2, 4000 + 2000 119 / 112.  Two
+  // thirds of the share and half of it: 15360 + 9256 13% and 6% above the term's.
   if (U + U / 32 + 3 < kmax) U += U / 32 + 3;
   if (U < kMinChunkTiles) U = kMinChunkTiles;
   if ((kmax + U - 1) / U > kMaxChunks) U = (kmax + kMaxChunks - 1) / kMaxChunks;
@@ -299,17 +302,19 @@ __device__ __forceinline__ void hold_acc(f32x16 (&o)[N]) {
 //    has it redone;
 //  - an MFMA leaves room for about five other instructions (measured: 32.9 cycles with
 //    four, 44 with eight, 5 each beyond), so the rest is dealt out between the MFMAs;
-//  - the tile moves are LDS DMA (no registers, no ds_write), one beside every eighth
-//    MFMA: issued together they cost 900 cycles a tile, spread about 170;
+//  - the tile moves are LDS DMA (no registers, no ds_write), one beside every fourth MFMA
+//    of QK (every second with NB = 1): issued together they cost 900 cycles a tile, spread
+//    about 170;
 //  - rare blocks (mask, moved reference, ragged tiles) are marked unlikely, so that the
 //    loop is one run of code: in line they cost 800 of 3900 cycles a tile.
-// Per K/V operand read from LDS NB MFMAs run.  15360 + 9256 tokens, 6 heads: 3150 cycles
-// per 256 rows x 32 keys (2048 of MFMA) at the 1.9 GHz the power allows.  The call with
-// its other launches: 1900 us before (four waves of 32 rows, tiles through registers, one
-// phase after the other), 1230 us now, 0.92 PFLOP/s; a large library bf16 product reaches
+// Per K/V operand read from LDS NB MFMAs run.  15360 + 9256 tokens, 6 heads: 2.12 M cycles
+// (1.04 to 1.1 ms at the 1.9 to 2.0 GHz the power allows), which is 3800 per 256 rows x 32
+// keys of its longest units (558 key tiles), 2048 of them MFMA.  The layer's call with its
+// other launches: 1880 us before (four waves of 32 rows, tiles through registers, one phase
+// after the other), 1155 to 1200 us now, 0.98 PFLOP/s; a large library bf16 product reaches
 // 1.2 to 1.36 on this card.
 template <int D, int QT, int NB>
-__global__ __launch_bounds__(kThreads, prefill_wgs(D, NB)) void prefill_kernel(PrefillParams P) {
+__global__ __launch_bounds__(kThreads, prefill_wgs(D)) void prefill_kernel(PrefillParams P) {
   using QV = typename QVec<QT>::type;    // one MFMA operand in the query dtype
   const oscar_prefill_args_v1& A = P.a;
   const int tid = threadIdx.x, lane = tid & 63;

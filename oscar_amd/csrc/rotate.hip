@@ -105,8 +105,8 @@ __global__ __launch_bounds__(256) void rotate_kernel(oscar_rotate_args_v1 a) {
 // the whole contraction in registers (128 at D = 256, loaded once), the tile's rows are split
 // into hi and lo planes in LDS once for all waves, and the next tile's rows are in flight
 // beside the products.  rotate_kernel reads a row tile once per column block and R once per
-// 32 x 32 outputs: 55536 x 256 fp32 rows 108 us there, 31.6 us here (85 MB, 17 us at the
-// rate of a large copy; 48 MFMAs per wave and tile, 1.4 us).
+// 32 x 32 outputs: 55536 x 256 fp32 rows to bf16 101 us there, 28 us here (85 MB, 17 us at
+// the rate of a large copy; 48 MFMAs per wave and tile, 1.4 us).
 constexpr int kBigThreads = 512;
 constexpr int64_t kBigGrid = 256;  // one workgroup per compute unit
 // rotate_rows_kernel from this many bytes of x on: its workgroups first take all of R, which
