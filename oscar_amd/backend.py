@@ -40,7 +40,7 @@ MAX_DECODE_ROWS = 32  # rows (query tokens x heads per KV head) of one decode MF
 # sub-requests of MAX_DECODE_ROWS rows (each decodes the request's history once), up to
 # this many rows; longer chunks go to the MFMA prefill, which decodes the history once for
 # all.  The prefill is the faster one well below the line (6 heads of 256, split-K / prefill
-# in us: 400 tokens over 15000 132 / 141, 800 284 / 178, 2700 772 / 391), but its history V
+# in us: 400 tokens over 15000 131 / 130, 800 284 / 155, 2700 768 / 392), but its history V
 # values are rounded to bf16 and the split-K decode's are not: single outputs move by up to
 # 0.34 of the outputs' root mean square where a chunk changes route.
 MAX_SPLIT_ROWS = 32 * 512
